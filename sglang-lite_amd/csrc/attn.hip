@@ -19,22 +19,40 @@
 // One workgroup per (query token, group of 64 heads, split of the rows); a
 // small batch (decode) splits its rows over several workgroups so every CU
 // has one, and a second kernel merges the splits' partial maxima, sums and
-// outputs.  Eight wavefronts, two per SIMD: wavefront (hg, dq) owns heads
-// [32 hg, +32) of the group.  Per block of 64 rows:
-//   gather:  each wavefront dequantizes 8 rows (loaded during the previous
-//            block) into one row-major bf16 tile in LDS (swizzled);
-//   S^T = KV . Q^T (v_mfma_f32_32x32x16_bf16, Q^T fragments parked in LDS):
-//            wavefront dq = 2 dh + th the partial of the 32 tokens of half th
-//            over dims [256 dh, +256); the partials meet in LDS and each of
-//            the group's four wavefronts sums and finishes the softmax
-//            (identically);
-//   O^T += V^T . P^T: P^T is the S^T accumulator itself, cast to bf16 (the
-//            32x32 output layout of S^T is the B operand layout of the next
-//            MFMA), and V^T fragments come straight from the row-major tile
-//            with ds_read_b64_tr_b16, so no transposed copy is stored; each
-//            wavefront its 128 dims [128 dq, +128) over all 64 tokens.
-// In both products lane (head c, half g) owns head c: the running max, sum
-// and rescale factor of a head live in the lanes that hold its outputs.
+// outputs.  The split's valid indices are packed into a list in LDS first, so
+// masked entries (-1 pads of a short context, a prefill's early queries) cost
+// nothing.  Eight wavefronts in two roles, one of each per SIMD, so one
+// role's MFMAs fill the other's waits; the roles run blocks of 32 rows in
+// phases with one barrier each, S^T of block j + 1 beside O^T of block j:
+//   gather:  wavefronts 4-7, 8 rows each, into a ring of four 32 KB row-major
+//            bf16 tiles: bf16 rows by LDS DMA two phases ahead; FP8 rows into
+//            registers a phase ahead, then dequantized and stored;
+//   S^T = KV . Q^T (v_mfma_f32_16x16x32_bf16), wavefronts 0-3: wavefront
+//            (hh, th) 16 tokens x 32 heads over all 512 dims, its Q^T
+//            fragments (128 registers) loaded once, so no partial sums meet;
+//   P:       exp2 against the head's running reference, bf16, into one of two
+//            4 KB LDS tiles.  The reference moves only when a score exceeds it
+//            by more than 8 (log2 units), so as a rule no maxima are
+//            exchanged: a wavefront that sees such a score raises a flag, and
+//            only then the block's maxima meet in LDS and P and the
+//            accumulators are brought to the new reference;
+//   O^T += V^T . P^T (v_mfma_f32_32x32x16_bf16), wavefronts 4-7: wavefront w
+//            128 dims of all 64 heads (128 registers), V^T fragments by
+//            ds_read_b64_tr_b16 straight from the row-major tile, each of its
+//            bytes read once.
+// What bounds it: LDS traffic and MFMA issue, about evenly: per 32 rows the
+// LDS takes 32 KB of tile writes, 64 KB of S^T reads, 32 KB (at half rate) of
+// V^T reads and 16 KB of P reads; each SIMD 1024 cycles of MFMA (0.7 of the
+// 1.1 us a block takes), and a workgroup fills a CU, so its first loads and
+// its output rows (about 7 us a query) stand alone.  256 queries x 640 /
+// 2048 rows of a bf16 cache 45.9 / 113 -> 34.2 / 81 us against the version
+// before (one role, S^T over split dims with partial sums through LDS, 64-row
+// blocks), packed pages 53 / 133 -> 41.5 / 105; a 2048-token prefill chunk
+// (640 indices, -1 where a token has fewer rows) 320 -> 182 us.  The roles
+// without the MFMAs between reads and gathers (each fragment read waited for
+// by itself): 1.3 us a block.
+#include <algorithm>
+
 #include "sgl_common.h"
 #include "sgl_numeric.h"
 
@@ -43,7 +61,7 @@ namespace {
 
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef short v4s __attribute__((ext_vector_type(4)));
-typedef short v8s __attribute__((ext_vector_type(8)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef v4s __attribute__((address_space(3))) lds_v4s;
 
@@ -89,303 +107,571 @@ __device__ __forceinline__ uint32_t cvt2_e4m3_bf16(uint32_t w, float sc) {
   return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, sc, HI));
 }
 
-template <int FMT>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void sparse_attn_kernel(const AttnArgs a) {
-  __shared__ __align__(16) uint8_t sKV[kBlk * 1024];
-  __shared__ __align__(16) uint4 sQ[2][2][16][64];   // Q^T fragments, [hg][dh][ks][lane]
-  __shared__ __align__(16) float4 sS[8][4][64];      // S^T partials, [wave][quad][lane]
+// 16 bytes at an 8-byte aligned address (layout A rows)
+struct __attribute__((packed, aligned(8))) U4a8 {
+  uint32_t x, y, z, w;
+};
 
+// Barrier behind this wavefront's own LDS traffic and, with VM, its DMAs
+// (which the compiler does not count).  The register loads the compiler
+// counts stay in flight across the first form.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+__device__ __forceinline__ void dma_barrier() {
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// dma16v when j < n: a branch inside the asm, so that the code around it
+// stays one scheduling region.
+__device__ __forceinline__ void dma16v_if(uint64_t addr, uint32_t lds, int j, int n) {
+  asm volatile("s_cmp_ge_i32 %2, %3\n\ts_cbranch_scc1 .Lno_dma%=\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\t"
+               "global_load_lds_dwordx4 %0, off\n.Lno_dma%=:"
+               :: "v"(addr), "s"(lds), "s"(j), "s"(n) : "memory", "scc");
+}
+
+constexpr int kRows = 32;            // rows of a block (one phase)
+constexpr int kTile = kRows * 1024;  // bytes of a row-major bf16 tile
+constexpr int kRing = 4;             // tiles
+constexpr int kPTile = kHG * 64;     // bytes of P: [head][32 tokens] bf16
+
+// Selected rows held in LDS at a time (a multiple of 64): their addresses
+// and, FP8, the distance to their scale bytes.
+template <int FMT>
+constexpr int kList = FMT == SGL_ATTN_KV_BF16 ? 2752 : 1792;
+
+template <int FMT>
+struct Smem {
+  alignas(16) uint8_t kv[kRing * kTile];  // row tiles (Q, then outputs, pass through them)
+  alignas(16) uint8_t p[2 * kPTile];
+  alignas(16) uint64_t row[kList<FMT> + kRows];
+  uint32_t foot[FMT == SGL_ATTN_KV_BF16 ? 1 : kList<FMT> + kRows];
+  float mx[2][kHG];                       // block maxima per token half and head (then the sums)
+  float sink[kHG];                        // log2 units
+  int flag[4];                            // block n's at n % 4: a score above its reference
+};
+
+__device__ const uint4 g_zero_row[64] = {};  // what a block's rows past the list read
+
+// P [head h][32 tokens]: 16-byte chunk c (8 tokens) of row h.  The rotation
+// spreads 16 heads' reads of one chunk over all 64 banks.
+__device__ __forceinline__ uint32_t p_off(int h, int c) {
+  return (uint32_t)(h * 64 + ((c ^ ((h >> 2) & 3)) << 4));
+}
+
+// One role of the workgroup: S (wavefronts 0-3: scores and probabilities) or
+// not S (4-7: the outputs).  The two instantiations run the same sequence of
+// barriers; keeping them apart keeps the 128 registers of Q^T and the 128 of
+// O^T out of each other's wavefronts.
+// HT: 32-head tiles of the group that exist (1: at most 32 heads in all).
+template <int FMT, int HT, bool S>
+__device__ __forceinline__ void attn_role(const AttnArgs& a, Smem<FMT>& sm) {
+  constexpr bool kDma = FMT == SGL_ATTN_KV_BF16;
+  uint8_t* const sKV = sm.kv;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // wavefront (hg, dq): heads [32 hg, +32) of the group; S^T over dims
-  // [256 dh, +256) for tokens [32 th, +32) of a block (dq = 2 dh + th), and
-  // O^T over dims [128 dq, +128) for all 64 tokens
-  const int hg = wave & 1, dq = wave >> 1, dh = dq >> 1, th = dq & 1;
+  const int hh = (wave >> 1) & 1, th = wave & 1;  // S: heads [32 hh, +32), tokens [16 th, +16)
+  const int wo = wave & 3;                        // O: dims [128 wo, +128)
+  const int l16 = lane & 15, g4 = lane >> 4;
   const int g2 = lane >> 5, c32 = lane & 31;
-  const int64_t m = blockIdx.x, b = blockIdx.y;
+  // later queries of a prefill select more rows: they start first
+  const int64_t m = a.M - 1 - (int64_t)blockIdx.x, b = blockIdx.y;
   const int split = (int)(blockIdx.z % a.nsplit);
-  const int h0 = (int)(blockIdx.z / a.nsplit) * kHG + 32 * hg;  // this wavefront's first head
-  const bool active = h0 < a.Hh;
+  const int h0 = (int)(blockIdx.z / a.nsplit) * kHG;
+  const int nh = min(a.Hh - h0, kHG);             // heads of this group
+  const bool live = !S || 32 * hh < nh;           // S: this wavefront's heads exist
   const uint8_t* kvb = a.kv + b * a.kv_bstride;
   const int32_t* idxp = a.idx + (b * a.M + m) * a.K;
+  const uint32_t kv_lds = __builtin_amdgcn_readfirstlane(lds_u32(sKV));
 
-  // S^T A operand: token 32 th + c32, chunk 32 dh + 2 ks + g2; the swizzle
-  // only touches the chunk's low four bits, so ks % 8 picks one of eight
-  // bases and the rest is an immediate offset
-  uint32_t qa[8];
+  // S^T operands: row l16 (a token, or a head), chunk 4 kk + g4; the swizzle
+  // only touches the chunk's low four bits, so kk % 4 picks one of four bases
+  // and the rest is an immediate offset
+  uint32_t ka[4];
 #pragma unroll
-  for (int k8 = 0; k8 < 8; ++k8)
-    qa[k8] = (32 * th + c32) * 1024 + 512 * dh + ((((2 * k8 + g2) ^ sw(c32)) & 15) << 4);
-  // V^T A operand by transpose read: in each 16-lane group G, source lane s
-  // reads 4 dims of token 16 s4 + 8 e + 4 (G >> 1) + (s >> 2), and the read
-  // hands each lane 4 consecutive tokens of one dim, i.e. 4 consecutive K
-  // elements of one row of V^T.  Bases for each (e, dt).
-  uint32_t va[2][4];
-  {
-    const int G = lane >> 4, s16 = lane & 15;
+  for (int k4 = 0; k4 < 4; ++k4) ka[k4] = l16 * 1024 + (((4 * k4 + g4) ^ sw(l16)) << 4);
+  // V^T operand by transpose read: in each 16-lane group G, source lane s
+  // reads 4 dims of token 16 s4 + 8 (G >> 1) + 4 e + (s >> 2), and the read
+  // hands each lane 4 consecutive tokens of one dim; e = 0, 1 give the lane's
+  // 8 consecutive K elements.  Bases for each e; dim tile dt is chunk 4 dt of
+  // the lane's low four chunk bits, which the swizzle only xors.
+  uint32_t va[2];
 #pragma unroll
-    for (int e = 0; e < 2; ++e)
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt) {
-        const int tok = 8 * e + 4 * (G >> 1) + (s16 >> 2);
-        const int cl = 4 * dt + 2 * (G & 1) + ((s16 & 3) >> 1);
-        va[e][dt] = tok * 1024 + 256 * dq + ((cl ^ sw(tok)) << 4) + 8 * (s16 & 1);
-      }
+  for (int e = 0; e < 2; ++e) {
+    const int tok = 8 * (g4 >> 1) + 4 * e + (l16 >> 2);
+    const int cl = 16 * wo + 2 * (g4 & 1) + ((l16 & 3) >> 1);
+    va[e] = tok * 1024 + ((cl ^ sw(tok)) << 4) + 8 * (l16 & 1);
   }
 
-  v16f acc[4];
-#pragma unroll
-  for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[dt][r] = 0.0f;
   const float NEG_INF = -__builtin_huge_valf();
   const float c1 = a.scale * kLog2e;
-  float m_run = NEG_INF, l_run = 0.0f;  // head c32: reference point (log2 units) and sum
-
-  // layout A per-lane byte offsets: lanes < 56 take 8 e4m3 bytes and the
-  // row's 8-byte scale footer, lanes 56..63 the 16 rope bytes in two halves
-  const bool nope_lane = lane < 56;
-  const uint32_t o0 = nope_lane ? 8 * lane : kANope + 16 * (lane - 56);
-  const uint32_t o1r = kANope + 8 + 16 * (lane - 56);  // rope second half (rope lanes)
-  const int sb_shift = 8 * ((lane >> 3) & 3);
-  const bool sb_hi = (lane >> 3) >= 4;
-
-  // A block's indices are loaded unconditionally (clamped to the last one)
-  // and checked where they are used: the check waits for the load, and since
-  // loads complete in order, a check right after the load would also wait
-  // for every row gather issued before it.
-  auto load_ids = [&](int j) -> int32_t {
-    const int64_t p = (int64_t)j * kBlk + lane;
-    return idxp[p < a.K ? p : a.K - 1];
-  };
-  auto check_id = [&](int j, int32_t id) -> int32_t {
-    const int64_t p = (int64_t)j * kBlk + lane;
-    return (p < a.K && id >= 0 && id < a.n) ? id : -1;
-  };
-  // this wavefront's 8 rows of the block: tokens 8 wave + rr.  The gathers
-  // are unconditional (a missing row reads row 0, which store_rows zeroes),
-  // so no branch splits the loads and the compiler's wait before the stores
-  // counts the loads in flight instead of draining them.
-  uint4 raw[8];
-  auto load_rows = [&](int32_t ids) {
-    if (a.n == 0) return;  // no rows at all: store_rows zeroes every row
-#pragma unroll
-    for (int rr = 0; rr < 8; ++rr) {
-      const int idr = __builtin_amdgcn_readlane(ids, 8 * wave + rr);
-      const int id = idr >= 0 ? idr : 0;
-      uint4 v;
-      {
-        if constexpr (FMT == SGL_ATTN_KV_BF16) {
-          v = *reinterpret_cast<const uint4*>(kvb + (int64_t)id * a.ld * 2 + lane * 16);
-        } else {
-          const uint8_t* data;
-          const uint8_t* foot;
-          if constexpr (FMT == SGL_ATTN_KV_A_PAGED) {
-            const int pg = a.page_shift >= 0 ? id >> a.page_shift : (int)((uint32_t)id / (uint32_t)a.page);
-            const int l = id - pg * a.page;
-            const uint8_t* pbase = kvb + (int64_t)pg * a.page * kARow;
-            data = pbase + l * kAData;
-            foot = pbase + a.page * kAData + l * 8;
-          } else {
-            data = kvb + (int64_t)id * kARow;
-            foot = data + kAData;
-          }
-          const uint2 x = *reinterpret_cast<const uint2*>(data + o0);
-          const uint2 y = *reinterpret_cast<const uint2*>(nope_lane ? foot : data + o1r);
-          v = make_uint4(x.x, x.y, y.x, y.y);
-        }
-      }
-      raw[rr] = v;
-    }
-  };
-  auto store_rows = [&](int32_t ids) {
-#pragma unroll
-    for (int rr = 0; rr < 8; ++rr) {
-      uint4 v = raw[rr];
-      if (__builtin_amdgcn_readlane(ids, 8 * wave + rr) < 0) v = make_uint4(0, 0, 0, 0);
-      if constexpr (FMT != SGL_ATTN_KV_BF16) {
-        const uint32_t word = sb_hi ? v.w : v.z;
-        const float sc = bits_f32(((word >> sb_shift) & 0xFFu) << 23);  // 2^(e8m0 - 127)
-        // word by word: a select of whole uint4 values goes through scratch
-        const uint32_t c0 = cvt2_e4m3_bf16<false>(v.x, sc), c1 = cvt2_e4m3_bf16<true>(v.x, sc);
-        const uint32_t c2 = cvt2_e4m3_bf16<false>(v.y, sc), c3 = cvt2_e4m3_bf16<true>(v.y, sc);
-        v.x = nope_lane ? c0 : v.x;
-        v.y = nope_lane ? c1 : v.y;
-        v.z = nope_lane ? c2 : v.z;
-        v.w = nope_lane ? c3 : v.w;
-      }
-      const int t = 8 * wave + rr;
-      *reinterpret_cast<uint4*>(sKV + t * 1024 + ((lane ^ sw(t)) << 4)) = v;
-    }
-  };
-
-  const int nblk_all = (int)((a.K + kBlk - 1) / kBlk);
-  const int jb = split * a.bps;  // this split's first block
-  const int nblk = jb + a.bps < nblk_all ? jb + a.bps : nblk_all;
-  // indices run two blocks ahead of the MFMAs, the rows one block ahead;
-  // past the last block the loads repeat it (their results are unused)
-  int32_t ids = jb < nblk ? check_id(jb, load_ids(jb)) : -1;
-  int32_t ids_next = jb < nblk ? load_ids(jb + 1 < nblk ? jb + 1 : jb) : -1;  // raw (none when K == 0)
-  load_rows(ids);
-  // Q^T B operand: lane (head c32, half g2) of step ks holds
-  // q[h0 + c32][256 dh + 16 ks + 8 g2, +8); the two token halves share it.
-  // Loaded after the first rows' gathers are issued, so its memory latency
-  // overlaps theirs: the first block waits for two memory round trips (the
-  // indices, then the rows with Q), not three
-  {
-    const int h = min(h0 + c32, a.Hh - 1);
-    const uint16_t* qrow = a.q + ((b * a.M + m) * a.Hh + h) * (int64_t)kD + 256 * dh + 8 * g2;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const int ks = 8 * th + k;
-      sQ[hg][dh][ks][lane] = *reinterpret_cast<const uint4*>(qrow + 16 * ks);
-    }
-  }
-  for (int j = jb; j < nblk; ++j) {
-    const uint64_t valid = __ballot(ids >= 0);
-    __syncthreads();  // the previous block's tile is consumed
-    store_rows(ids);
-    __syncthreads();  // block j (and, the first time, Q) is in LDS
-    {
-      const int jn = j + 1 < nblk ? j + 1 : j;
-      ids = j + 1 < nblk ? check_id(jn, ids_next) : -1;
-      ids_next = load_ids(j + 2 < nblk ? j + 2 : jn);  // before the rows it would wait behind
-      load_rows(ids);
-    }
-    if (!active) {
-      __syncthreads();  // (partials exchanged)
-      continue;
-    }
-    // partial S^T of tile th over dims [256 dh, +256): lane (head c32, g2)
-    // gets token 32 th + 8 (r / 4) + 4 g2 + r % 4 in sp[r]
-    v16f sp;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) sp[r] = 0.0f;
-#pragma unroll
-    for (int ks = 0; ks < 16; ++ks) {
-      const v8bf qf = __builtin_bit_cast(v8bf, sQ[hg][dh][ks][lane]);
-      const v8bf kvf = *reinterpret_cast<const v8bf*>(sKV + qa[ks & 7] + 256 * (ks >> 3));
-      sp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kvf, qf, sp, 0, 0, 0);
-    }
-#pragma unroll
-    for (int q4 = 0; q4 < 4; ++q4)
-      sS[wave][q4][lane] = make_float4(sp[4 * q4], sp[4 * q4 + 1], sp[4 * q4 + 2], sp[4 * q4 + 3]);
-    __syncthreads();  // partials exchanged
-    // full S^T of both tiles: tile tt = partial (dh 0) + partial (dh 1), the
-    // same sum in each of the head group's four wavefronts
-    v16f s[2];
-#pragma unroll
-    for (int tt = 0; tt < 2; ++tt) {
-      const int w0 = hg + 2 * tt, w1 = hg + 4 + 2 * tt;  // (hg, dh = 0 / 1, th = tt)
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const float4 x = sS[w0][q4][lane], y = sS[w1][q4][lane];
-        s[tt][4 * q4] = x.x + y.x;
-        s[tt][4 * q4 + 1] = x.y + y.y;
-        s[tt][4 * q4 + 2] = x.z + y.z;
-        s[tt][4 * q4 + 3] = x.w + y.w;
-      }
-    }
-    if (valid != ~0ull) {
-      const uint64_t vl = g2 ? (valid >> 4) : valid;
-#pragma unroll
-      for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          if (!((vl >> (32 * tt + 8 * (r >> 2) + (r & 3))) & 1ull)) s[tt][r] = NEG_INF;
-    }
-    // online softmax of head c32 (scale > 0: max(s) * c1 = max(s * c1))
-    float mx = NEG_INF;
-#pragma unroll
-    for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) mx = __builtin_fmaxf(mx, s[tt][r]);
-    mx = __builtin_fmaxf(mx, __shfl_xor(mx, 32, 64));
-    // The reference point moves only when the block maximum exceeds it by
-    // more than 8 (log2 units): the probabilities stay <= 256 (exact range
-    // in bf16, same relative rounding) and the accumulator is rarely
-    // rescaled.  Any reference >= the running max gives the same softmax.
-    const float m_blk = mx * c1;
-    const bool move = !(m_blk <= m_run + 8.0f);  // also true while m_run = -inf
-    const float m_new = move ? __builtin_fmaxf(m_run, m_blk) : m_run;
-    const float ref = m_new == NEG_INF ? 0.0f : m_new;  // a fully masked prefix keeps o = 0
-    const float alpha = move ? __builtin_amdgcn_exp2f(m_run - ref) : 1.0f;
-    float ls = 0.0f;
-#pragma unroll
-    for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[tt][r], c1, -ref));
-        ls += p;
-        s[tt][r] = p;
-      }
-    ls += __shfl_xor(ls, 32, 64);
-    l_run = l_run * alpha + ls;
-    m_run = m_new;
-    // P^T B operands: K step s4 (16 tokens) = tile s4 / 2, registers 8 (s4 % 2) + e
-    v8bf pb[4];
-#pragma unroll
-    for (int s4 = 0; s4 < 4; ++s4) {
-      v8s w;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint32_t pk = pk2_bf16(s[s4 >> 1][8 * (s4 & 1) + 2 * e], s[s4 >> 1][8 * (s4 & 1) + 2 * e + 1]);
-        w[2 * e] = (short)(pk & 0xFFFFu);
-        w[2 * e + 1] = (short)(pk >> 16);
-      }
-      pb[s4] = __builtin_bit_cast(v8bf, w);
-    }
-    if (j > jb && __ballot(alpha != 1.0f)) {  // (the accumulator is zero before the first block)
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[dt][r] *= alpha;
-    }
-    // O^T += V^T . P^T over this wavefront's 4 tiles of 32 dims (K step
-    // outer: four independent accumulators between dependent MFMAs)
-#pragma unroll
-    for (int s4 = 0; s4 < 4; ++s4) {
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt) {
-        const v4s lo = lds_tr16(sKV, va[0][dt] + 16384 * s4);
-        const v4s hi = lds_tr16(sKV, va[1][dt] + 16384 * s4);
-        const v8bf vf = __builtin_bit_cast(v8bf, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pb[s4], acc[dt], 0, 0, 0);
-      }
-    }
-  }
-  if (!active) return;
-  const int h = h0 + c32;
-  if (h >= a.Hh) return;
-  // lane (head h, g2) holds dims 128 dq + 32 dt + 8 (r / 4) + 4 g2 + r % 4 in acc[dt][r]
-  if (a.nsplit > 1) {
-    const int64_t qs = (b * a.M + m) * a.nsplit + split;
-    if (dq == 0 && g2 == 0) {
-      float* ml = a.ws_ml + (qs * a.Hh + h) * 2;
-      ml[0] = m_run;
-      ml[1] = l_run;
-    }
-    float* row = a.ws_acc + (qs * a.Hh + h) * (int64_t)kD + 128 * dq + 4 * g2;
+  // reference points (log2 units): S: of heads 32 hh + 16 i + l16, with this
+  // lane's share (its tokens) of their sums; O: of heads 32 i + c32
+  float mref[2] = {NEG_INF, NEG_INF}, lsum[2] = {0.0f, 0.0f};
+  // S: what the exponentials subtract (a fully masked prefix keeps o = 0) and
+  // the raw score from which the reference has to move
+  float nref[2] = {0.0f, 0.0f}, lim[2] = {NEG_INF, NEG_INF};
+  v8bf qf[S ? 2 : 1][S ? 16 : 1];  // Q^T fragments: [head tile][32-dim step]
+  v4f st[2];                       // S: scores of the last block
+  v16f acc[S ? 1 : 4][S ? 1 : HT];  // O^T: [32-dim tile][32-head tile]
+  if constexpr (!S) {
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4)
-        *reinterpret_cast<float4*>(row + 32 * dt + 8 * q4) =
-            make_float4(acc[dt][4 * q4], acc[dt][4 * q4 + 1], acc[dt][4 * q4 + 2], acc[dt][4 * q4 + 3]);
-    return;
+      for (int ht = 0; ht < HT; ++ht)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[dt][ht][r] = 0.0f;
   }
-  // o = acc / (l + exp(sink - m))
-  const float ref = m_run == NEG_INF ? 0.0f : m_run;
-  const float inv = 1.0f / (l_run + __builtin_amdgcn_exp2f(a.sink[h] * kLog2e - ref));
-  uint16_t* orow = a.o + ((b * a.M + m) * a.Hh + h) * (int64_t)kD + 128 * dq + 4 * g2;
+
+  // the sinks, fetched long before they are used
+  if (S && wave == 0 && lane < nh) sm.sink[lane] = a.sink[h0 + lane] * kLog2e;
+
+  const int nblk_all = (int)((a.K + kBlk - 1) / kBlk);
+  const int jb = split * a.bps;  // this split's first 64 indices
+  const int64_t k_begin = (int64_t)jb * kBlk;
+  const int64_t k_end = min((int64_t)min(jb + a.bps, nblk_all) * kBlk, a.K);
+
+  bool first = true;
+  for (int64_t kc = k_begin; kc < k_end || first; kc += kList<FMT>) {
+    // ---- the chunk's valid rows, packed in order, padded to a whole block.
+    // Every wavefront writes the whole list (the same values), so each reads
+    // back its own writes
+    if (!first) __syncthreads();  // the previous chunk's list and tiles are consumed
+    if (threadIdx.x < 4) sm.flag[threadIdx.x] = 0;
+    int cnt = 0;
+    const int64_t ke = min(kc + (int64_t)kList<FMT>, k_end);
+    auto put_row = [&](int at, int id) {
+      if constexpr (kDma) {
+        sm.row[at] = (uint64_t)(uintptr_t)kvb + (uint64_t)(uint32_t)id * ((uint64_t)a.ld * 2);
+      } else if constexpr (FMT == SGL_ATTN_KV_A_PAGED) {
+        const uint32_t pg = a.page_shift >= 0 ? (uint32_t)id >> a.page_shift : (uint32_t)id / (uint32_t)a.page;
+        const uint32_t l = (uint32_t)id - pg * (uint32_t)a.page;
+        sm.row[at] = (uint64_t)(uintptr_t)kvb + (uint64_t)pg * ((uint64_t)a.page * kARow) + l * (uint32_t)kAData;
+        sm.foot[at] = (uint32_t)a.page * kAData - l * (uint32_t)(kAData - 8);
+      } else {
+        sm.row[at] = (uint64_t)(uintptr_t)kvb + (uint64_t)(uint32_t)id * kARow;
+        sm.foot[at] = kAData;
+      }
+    };
+    for (int64_t p0 = kc; p0 < ke; p0 += 4 * 64) {
+      int32_t id[4];
 #pragma unroll
-  for (int dt = 0; dt < 4; ++dt)
+      for (int u = 0; u < 4; ++u) {
+        const int64_t p = p0 + u * 64 + lane;
+        id[u] = idxp[p < ke ? p : ke - 1];
+      }
 #pragma unroll
-    for (int q4 = 0; q4 < 4; ++q4)
-      *reinterpret_cast<uint2*>(orow + 32 * dt + 8 * q4) =
-          make_uint2(pk2_bf16(acc[dt][4 * q4] * inv, acc[dt][4 * q4 + 1] * inv),
-                     pk2_bf16(acc[dt][4 * q4 + 2] * inv, acc[dt][4 * q4 + 3] * inv));
+      for (int u = 0; u < 4; ++u) {
+        const bool ok = p0 + u * 64 + lane < ke && id[u] >= 0 && id[u] < a.n;
+        const uint64_t mask = __ballot(ok);
+        const int before = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                                     __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
+        if (ok) put_row(cnt + before, id[u]);
+        cnt += __popcll(mask);
+      }
+    }
+    cnt = __builtin_amdgcn_readfirstlane(cnt);
+    if (lane < kRows) {  // (read only when cnt > 0: row 0 exists)
+      if constexpr (kDma) sm.row[cnt + lane] = (uint64_t)(uintptr_t)g_zero_row;
+      else put_row(cnt + lane, 0);
+    }
+    const int nblk = (cnt + kRows - 1) / kRows;
+
+    // ---- row gathers: rows 8 wo + rr of a block, by the O wavefronts (the
+    // first time the S wavefronts take block 1).  bf16: one DMA per row, lane
+    // i fetching the chunk that belongs at i.  FP8 (layout A): two rows a
+    // load, 28 lanes each 16 e4m3 bytes (lanes 56-63 repeat lane 55) and
+    // their scale byte, and one load for the 16-byte rope pieces of all eight
+    // rows (lane: row lane / 8, piece lane % 8).  (One row a load, 56 lanes x
+    // 8 bytes, with the scales passed between lanes, took three times the
+    // instructions: 2048 rows x 256 queries 118 us, this form 105)
+    int ln = lane;  // made opaque where the gathers run, so that their per-row offsets are formed there
+                    // and not kept in registers across the phases
+    auto dma_row = [&](int j, int rr, uint64_t row) {  // (a block past the last: nothing)
+      dma16v_if(row + (uint32_t)((ln ^ sw(8 * wo + rr)) << 4),
+                kv_lds + (uint32_t)((j & (kRing - 1)) * kTile + wo * 8192 + rr * 1024), j, nblk);
+    };
+    struct Raw {  // FP8 rows on their way: two per pair
+      U4a8 nope[kDma ? 1 : 4], rope;
+      uint32_t sc[kDma ? 1 : 4];
+    } raw;
+    auto load_pair = [&](int at, int p, Raw& w) {
+      const int lc = min(ln, 55), half = lc >= 28, piece = lc - 28 * half;
+      const uint64_t row = sm.row[at + 2 * p + half];
+      w.nope[p] = *reinterpret_cast<const U4a8*>((uintptr_t)(row + 16 * piece));
+      w.sc[p] = *reinterpret_cast<const uint8_t*>((uintptr_t)(row + sm.foot[at + 2 * p + half] + (piece >> 2)));
+    };
+    auto store_pair = [&](int j, int p, const Raw& w) {
+      const int lc = min(ln, 55), half = lc >= 28, piece = lc - 28 * half;
+      const uint32_t c = (uint32_t)(((2 * (p & 1)) << 2) | ((2 * wo + (p >> 1)) & 3));  // with half << 2: sw(row)
+      const uint32_t off = (uint32_t)((j & (kRing - 1)) * kTile + wo * 8192 + p * 2048) +
+                           ((uint32_t)(half * 1024 + ((2 * piece) ^ (half << 2)) * 16) ^ (c << 4));
+      const float sc = bits_f32(w.sc[p] << 23);  // 2^(e8m0 - 127)
+      const U4a8 x = w.nope[p];
+      *reinterpret_cast<uint4*>(sKV + off) =
+          make_uint4(cvt2_e4m3_bf16<false>(x.x, sc), cvt2_e4m3_bf16<true>(x.x, sc),
+                     cvt2_e4m3_bf16<false>(x.y, sc), cvt2_e4m3_bf16<true>(x.y, sc));
+      *reinterpret_cast<uint4*>(sKV + (off ^ 16)) =
+          make_uint4(cvt2_e4m3_bf16<false>(x.z, sc), cvt2_e4m3_bf16<true>(x.z, sc),
+                     cvt2_e4m3_bf16<false>(x.w, sc), cvt2_e4m3_bf16<true>(x.w, sc));
+    };
+    auto load_rope = [&](int at) -> U4a8 {
+      return *reinterpret_cast<const U4a8*>((uintptr_t)(sm.row[at + (ln >> 3)] + kANope + 16 * (ln & 7)));
+    };
+    auto store_rope = [&](int j, const U4a8& x) {  // then zeros for the rows past the list
+      const int t = 8 * wo + (ln >> 3);
+      uint8_t* tile = sKV + (j & (kRing - 1)) * kTile;
+      *reinterpret_cast<uint4*>(tile + t * 1024 + (((56 + (ln & 7)) ^ sw(t)) << 4)) = make_uint4(x.x, x.y, x.z, x.w);
+      const int left = cnt - j * kRows - 8 * wo;
+      if (left < 8)
+        for (int rr = max(left, 0); rr < 8; ++rr)
+          *reinterpret_cast<uint4*>(tile + (8 * wo + rr) * 1024 + lane * 16) = make_uint4(0, 0, 0, 0);
+    };
+    asm volatile("" : "+v"(ln));
+    {
+      const int j = S ? 1 : 0, at = j * kRows + 8 * wo;
+      if (j < nblk) {
+        if constexpr (kDma) {
+#pragma unroll
+          for (int rr = 0; rr < 8; ++rr) dma_row(j, rr, sm.row[at + rr]);
+        } else {
+#pragma unroll
+          for (int p = 0; p < 4; ++p) load_pair(at, p, raw);
+          raw.rope = load_rope(at);
+        }
+      }
+      if (first) {
+        // Q rows through the last two tiles: one DMA per head row
+#pragma unroll
+        for (int rr = 0; rr < 8; ++rr) {
+          const int h = 8 * wave + rr;
+          const uint8_t* row = reinterpret_cast<const uint8_t*>(
+              a.q + ((b * a.M + m) * a.Hh + h0 + min(h, nh - 1)) * (int64_t)kD);
+          dma16(row, (uint32_t)((lane ^ sw(h)) << 4), kv_lds + (uint32_t)(2 * kTile + h * 1024));
+        }
+      }
+      if constexpr (!kDma) {
+        if (j < nblk) {
+#pragma unroll
+          for (int p = 0; p < 4; ++p) store_pair(j, p, raw);
+          store_rope(j, raw.rope);
+        }
+      }
+    }
+    dma_barrier();  // tiles 0 and 1, and Q, are whole
+    if (first) {
+      if constexpr (S) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int kk = 0; kk < 16; ++kk)
+            qf[i][kk] = *reinterpret_cast<const v8bf*>(sKV + 2 * kTile + (32 * hh + 16 * i) * 1024 +
+                                                       ka[kk & 3] + 256 * (kk >> 2));
+      }
+      lds_barrier();  // Q is out of the tiles
+      first = false;
+    }
+
+    // S: P of this lane's tokens of block n against the current references
+    float ls[2] = {0.0f, 0.0f};
+    auto put_p = [&](int n) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        float p[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) p[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(st[i][r], c1, nref[i]));
+        ls[i] = (p[0] + p[1]) + (p[2] + p[3]);
+        *reinterpret_cast<uint2*>(sm.p + (n & 1) * kPTile + p_off(32 * hh + 16 * i + l16, 2 * th + (g4 >> 1)) +
+                                  8 * (g4 & 1)) = make_uint2(pk2_bf16(p[0], p[1]), pk2_bf16(p[2], p[3]));
+      }
+    };
+    // Block n has a score above its head's reference: the reference of a head
+    // moves to its block maximum where that exceeds it by more than 8 (log2
+    // units): the probabilities stay <= 256 (exact range in bf16, same
+    // relative rounding).  Any reference gives the same softmax.  Both roles
+    // come here, the S wavefronts with block n's scores in st.
+    auto move_refs = [&](int n) {
+      if constexpr (S) {
+        if (live) {
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            float mx = __builtin_fmaxf(__builtin_fmaxf(st[i][0], st[i][1]), __builtin_fmaxf(st[i][2], st[i][3]));
+            mx = __builtin_fmaxf(mx, __shfl_xor(mx, 16, 64));
+            mx = __builtin_fmaxf(mx, __shfl_xor(mx, 32, 64));
+            if (g4 == 0) sm.mx[th][32 * hh + 16 * i + l16] = mx;
+          }
+        }
+      }
+      lds_barrier();  // maxima exchanged
+      float f[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int h = S ? 32 * hh + 16 * i + l16 : 32 * i + c32;
+        const float mx = __builtin_fmaxf(sm.mx[0][h], sm.mx[1][h]) * c1;  // (scale > 0)
+        const float mn = !(mx <= mref[i] + 8.0f) ? __builtin_fmaxf(mref[i], mx) : mref[i];
+        f[i] = mn == mref[i] ? 1.0f : __builtin_amdgcn_exp2f(mref[i] - (mn == NEG_INF ? 0.0f : mn));
+        mref[i] = mn;
+      }
+      if constexpr (S) {
+        if (live) {
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            lsum[i] *= f[i];
+            nref[i] = mref[i] == NEG_INF ? 0.0f : -mref[i];
+            lim[i] = (mref[i] + 8.0f) / c1;
+          }
+          put_p(n);
+        }
+      } else {
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+          for (int ht = 0; ht < HT; ++ht)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[dt][ht][r] *= f[ht];
+      }
+      lds_barrier();  // P rewritten
+    };
+
+    // ---- phases: in phase j S^T and P of block j + 1 beside O^T of block j,
+    // one barrier after each.  A phase's first reads go out before the flag of
+    // block j is looked at
+    if constexpr (S) {
+      for (int j = -1; j < nblk; ++j) {
+        const int n = j + 1;
+        const uint8_t* tile = sKV + (n & (kRing - 1)) * kTile + 16 * th * 1024;
+        // four groups of four 32-dim steps, each group's fragments read while
+        // the one before is multiplied (left to itself the compiler reads one
+        // fragment, waits for it and multiplies)
+        v8bf kvf[2][4];
+        auto read4 = [&](int g) {
+#pragma unroll
+          for (int k4 = 0; k4 < 4; ++k4)
+            kvf[g & 1][k4] = *reinterpret_cast<const v8bf*>(tile + ka[k4] + 256 * g);
+        };
+        const int flag = sm.flag[j & 3];
+        read4(0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (j >= 0) {
+          if (__builtin_amdgcn_readfirstlane(flag)) move_refs(j);
+          lsum[0] += ls[0];
+          lsum[1] += ls[1];
+        }
+        if (threadIdx.x == 0) sm.flag[(j + 2) & 3] = 0;
+        if (n < nblk && live) {
+          // lane (head l16, g4) gets tokens 16 th + 4 g4 + r
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) st[i][r] = 0.0f;
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            if (g < 3) read4(g + 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int k4 = 0; k4 < 4; ++k4)
+#pragma unroll
+              for (int i = 0; i < 2; ++i)
+                st[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kvf[g & 1][k4], qf[i][4 * g + k4], st[i], 0, 0, 0);
+          }
+          if (cnt - n * kRows < kRows) {
+            const int left = cnt - n * kRows - 16 * th - 4 * g4;  // this lane's tokens past it are masked
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (r >= left) st[0][r] = st[1][r] = NEG_INF;
+          }
+          bool over = false;  // (also while the reference is -inf)
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+            over |= !(__builtin_fmaxf(__builtin_fmaxf(st[i][0], st[i][1]),
+                                      __builtin_fmaxf(st[i][2], st[i][3])) <= lim[i]);
+          if (__ballot(over) && lane == 0) sm.flag[n & 3] = 1;
+          put_p(n);
+        }
+        lds_barrier();
+      }
+    } else {
+      // the rows of block 2
+      uint64_t row_next[kDma ? 8 : 1];  // bf16: the addresses of the next eight rows
+      auto list_at = [&](int j) -> int { return min(j, nblk - 1) * kRows + 8 * wo; };
+      auto read_rows = [&](int j) {
+        if constexpr (kDma) {
+#pragma unroll
+          for (int rr = 0; rr < 8; rr += 2) {
+            const ulonglong2 v = *reinterpret_cast<const ulonglong2*>(&sm.row[list_at(j) + rr]);
+            row_next[rr] = v.x;
+            row_next[rr + 1] = v.y;
+          }
+        }
+      };
+      if (nblk > 0) {
+        read_rows(2);
+        if constexpr (kDma) {
+#pragma unroll
+          for (int rr = 0; rr < 8; ++rr) dma_row(2, rr, row_next[rr]);
+        } else {
+#pragma unroll
+          for (int p = 0; p < 4; ++p) load_pair(list_at(2), p, raw);
+          raw.rope = load_rope(list_at(2));
+        }
+      }
+      lds_barrier();  // (block 1's tile, the first time whole, is S's next)
+      for (int j = 0; j < nblk; ++j) {
+        const uint8_t* tile = sKV + (j & (kRing - 1)) * kTile;
+        v8bf pf[2][HT], vf[2][4];
+        auto read_p = [&](int s4) {
+#pragma unroll
+          for (int ht = 0; ht < HT; ++ht)
+            pf[s4][ht] = *reinterpret_cast<const v8bf*>(sm.p + (j & 1) * kPTile + p_off(32 * ht + c32, 2 * s4 + g2));
+        };
+        auto read_v = [&](int s4) {
+#pragma unroll
+          for (int dt = 0; dt < 4; ++dt) {
+            const v4s lo = lds_tr16(tile, (va[0] ^ (dt << 6)) + 16384 * s4);
+            const v4s hi = lds_tr16(tile, (va[1] ^ (dt << 6)) + 16384 * s4);
+            vf[s4][dt] = __builtin_bit_cast(v8bf, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+          }
+        };
+        const int flag = sm.flag[j & 3];
+        if constexpr (!kDma) asm volatile("" : "+v"(va[0]), "+v"(va[1]));  // (the eight addresses: not kept)
+        read_p(0);
+        read_v(0);
+        read_rows(j + 3);
+        __builtin_amdgcn_sched_barrier(0);
+        if (__builtin_amdgcn_readfirstlane(flag)) {
+          move_refs(j);
+          read_p(0);
+        }
+        if constexpr (kDma) {  // (FP8: below, for want of registers)
+          read_p(1);
+          read_v(1);
+        }
+        asm volatile("" : "+v"(ln));
+        __builtin_amdgcn_sched_barrier(0);
+        // the MFMAs, and between them the gathers: bf16: block j + 3's DMAs,
+        // into the tile that held block j - 1; FP8: block j + 2's rows, loaded
+        // during the last phase, dequantized into their tile (past the last
+        // block, into a tile nobody reads), then block j + 3's loads
+#pragma unroll
+        for (int rr = 0; rr < 8; ++rr) {
+          const int s4 = rr >> 2, dt = rr & 3;
+          if constexpr (kDma) {
+            dma_row(j + 3, rr, row_next[rr]);
+          } else {
+            if (rr == 2) {
+              read_p(1);
+              read_v(1);
+            }
+            if (rr & 1)
+              load_pair(list_at(j + 3), rr >> 1, raw);
+            else
+              store_pair(j + 2, rr >> 1, raw);
+          }
+#pragma unroll
+          for (int ht = 0; ht < HT; ++ht)
+            acc[dt][ht] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[s4][dt], pf[s4][ht], acc[dt][ht], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (!kDma) {
+          store_rope(j + 2, raw.rope);
+          raw.rope = load_rope(list_at(j + 3));
+        }
+        // block j + 2's tile whole (block j + 3's eight DMAs may be in flight)
+        if constexpr (kDma) {
+          if (j + 3 < nblk)
+            asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+          else
+            dma_barrier();
+        } else {
+          lds_barrier();
+        }
+      }
+    }
+    if (kc >= k_end) break;  // no indices at all
+  }
+
+  // ---- the heads' sums meet in LDS; the outputs pass through the tiles so
+  // that they leave as whole rows
+  __syncthreads();
+  if constexpr (S) {
+    if (live) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        float l = lsum[i];
+        l += __shfl_xor(l, 16, 64);
+        l += __shfl_xor(l, 32, 64);
+        if (g4 == 0) sm.mx[th][32 * hh + 16 * i + l16] = l;
+      }
+    }
+  }
+  __syncthreads();
+  const int64_t qm = b * a.M + m;
+  if constexpr (!S) {
+    // lane (head 32 ht + c32, g2) holds dims 128 wo + 32 dt + 8 q4 + 4 g2 + 0..3
+#pragma unroll
+    for (int ht = 0; ht < HT; ++ht) {
+      const int h = 32 * ht + c32;
+      if (h < nh) {
+        const float l = sm.mx[0][h] + sm.mx[1][h];
+        if (a.nsplit > 1) {
+          if (wo == 0 && g2 == 0) {
+            float* ml = a.ws_ml + ((qm * a.nsplit + split) * a.Hh + h0 + h) * 2;
+            ml[0] = mref[ht];
+            ml[1] = l;
+          }
+#pragma unroll
+          for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+            for (int q4 = 0; q4 < 4; ++q4) {
+              const int c = 32 * wo + 8 * dt + 2 * q4 + g2;
+              *reinterpret_cast<float4*>(sKV + h * 2048 + ((c ^ sw(h)) << 4)) =
+                  make_float4(acc[dt][ht][4 * q4], acc[dt][ht][4 * q4 + 1], acc[dt][ht][4 * q4 + 2],
+                              acc[dt][ht][4 * q4 + 3]);
+            }
+        } else {
+          // o = acc / (l + exp(sink - m))
+          const float ref = mref[ht] == NEG_INF ? 0.0f : mref[ht];
+          const float inv = 1.0f / (l + __builtin_amdgcn_exp2f(sm.sink[h] - ref));
+#pragma unroll
+          for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+            for (int q4 = 0; q4 < 4; ++q4) {
+              const int c = 16 * wo + 4 * dt + q4;
+              *reinterpret_cast<uint2*>(sKV + h * 1024 + ((c ^ sw(h)) << 4) + 8 * g2) =
+                  make_uint2(pk2_bf16(acc[dt][ht][4 * q4] * inv, acc[dt][ht][4 * q4 + 1] * inv),
+                             pk2_bf16(acc[dt][ht][4 * q4 + 2] * inv, acc[dt][ht][4 * q4 + 3] * inv));
+            }
+        }
+      }
+    }
+  }
+  __syncthreads();
+  for (int h = wave; h < nh; h += 8) {
+    if (a.nsplit > 1) {
+      float* row = a.ws_acc + ((qm * a.nsplit + split) * a.Hh + h0 + h) * (int64_t)kD;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int c = 64 * u + lane;
+        *reinterpret_cast<float4*>(row + 4 * c) =
+            *reinterpret_cast<const float4*>(sKV + h * 2048 + ((c ^ sw(h)) << 4));
+      }
+    } else {
+      uint16_t* row = a.o + (qm * a.Hh + h0 + h) * (int64_t)kD;
+      *reinterpret_cast<uint4*>(row + 8 * lane) =
+          *reinterpret_cast<const uint4*>(sKV + h * 1024 + ((lane ^ sw(h)) << 4));
+    }
+  }
+}
+
+template <int FMT, int HT>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void sparse_attn_kernel(const AttnArgs a) {
+  __shared__ Smem<FMT> sm;
+  static_assert(sizeof(sm) <= 160 * 1024, "the LDS of a CU");
+  if (threadIdx.x < 256)
+    attn_role<FMT, HT, true>(a, sm);
+  else
+    attn_role<FMT, HT, false>(a, sm);
 }
 
 // Merge of the per-split partials, one wavefront per (query, head), maxima in
@@ -439,21 +725,32 @@ __global__ __launch_bounds__(256) void sparse_attn_combine_kernel(const AttnArgs
   *reinterpret_cast<uint4*>(a.o + w * (int64_t)kD + lane * 8) = make_uint4(wv[0], wv[1], wv[2], wv[3]);
 }
 
-// Splits of the gathered rows: enough workgroups to give every CU one, at
-// most one split per 64-row block and at most 8 splits.
-int attn_splits(int64_t B, int64_t M, int Hh, int64_t K) {
+// Splits of the gathered rows: at most enough workgroups to give every CU one,
+// at most one split per 64-row block and kMaxSplits.  A split shortens the
+// serial chain of blocks but writes an fp32 partial of all its heads (128 KB
+// per 64 heads) that the merge reads back, so it is taken where the chain it
+// saves costs more than that.  In tenths of a us, fitted to 1 / 8 / 32 / 64
+// sequences x 128 ... 2048 rows with 1 to 8 splits: a 64-row block 18 (bf16)
+// or 24 (FP8), a merge 26 plus 0.8 per partial, at most 116.  (64 sequences x 128
+// rows: one split 11.7 us, two 22.7; 32 x 640: five 23.8, two 24.7, one 26.6.)
+int attn_splits(int64_t B, int64_t M, int Hh, int64_t K, bool fp8) {
   const int64_t wgs = B * M * ((Hh + kHG - 1) / kHG);
   const int64_t nblk = (K + kBlk - 1) / kBlk;
-  int64_t ns = (device_cu_count() + wgs - 1) / (wgs > 0 ? wgs : 1);
-  if (ns > nblk) ns = nblk;
-  // every split writes an fp32 partial of all its heads (128 KB per 64 heads)
-  // that the merge reads back: past 8 splits that traffic costs more than the
-  // parallelism gains (8 sequences x 2048 rows: 32 splits 45.7 us, 8 splits
-  // 38.3 us, measured)
-  if (ns > kMaxSplits) ns = kMaxSplits;
-  if (ns <= 1) return 1;
-  const int64_t bps = (nblk + ns - 1) / ns;
-  return (int)((nblk + bps - 1) / bps);  // no empty split
+  int64_t most = (device_cu_count() + wgs - 1) / (wgs > 0 ? wgs : 1);
+  if (most > nblk) most = nblk;
+  if (most > kMaxSplits) most = kMaxSplits;
+  int best = 1;
+  int64_t best_cost = nblk * (fp8 ? 240 : 180);
+  for (int64_t want = 2; want <= most; ++want) {
+    const int64_t bps = (nblk + want - 1) / want, ns = (nblk + bps - 1) / bps;  // no empty split
+    const int64_t parts = 8 * wgs * ns;
+    const int64_t cost = bps * (fp8 ? 240 : 180) + 260 + (parts < 900 ? parts : 900);
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = (int)ns;
+    }
+  }
+  return best;
 }
 
 }  // namespace
@@ -461,7 +758,8 @@ int attn_splits(int64_t B, int64_t M, int Hh, int64_t K) {
 
 extern "C" size_t sgl_sparse_attn_workspace_size(int64_t B, int64_t M, int Hh, int64_t K) {
   if (B <= 0 || M <= 0 || Hh <= 0 || K <= 0) return 0;
-  const int ns = sgl::attn_splits(B, M, Hh, K);
+  // enough for any kv_format
+  const int ns = std::max(sgl::attn_splits(B, M, Hh, K, false), sgl::attn_splits(B, M, Hh, K, true));
   if (ns == 1) return 0;
   return (size_t)(B * M * ns * Hh) * (sgl::kD + 2) * 4;
 }
@@ -502,7 +800,7 @@ extern "C" int sgl_sparse_attn(const void* q, int64_t B, int64_t M, int Hh, cons
   a.Hh = Hh;
   a.scale = softmax_scale;
   a.o = (uint16_t*)o;
-  a.nsplit = K > 0 ? sgl::attn_splits(B, M, Hh, K) : 1;
+  a.nsplit = K > 0 ? sgl::attn_splits(B, M, Hh, K, kv_format != SGL_ATTN_KV_BF16) : 1;
   const int64_t nblk = (K + sgl::kBlk - 1) / sgl::kBlk;
   a.bps = (int)((nblk + a.nsplit - 1) / a.nsplit);
   a.ws_acc = nullptr;
@@ -519,12 +817,21 @@ extern "C" int sgl_sparse_attn(const void* q, int64_t B, int64_t M, int Hh, cons
   }
   dim3 grid((unsigned)M, (unsigned)B, (unsigned)(((Hh + sgl::kHG - 1) / sgl::kHG) * a.nsplit));
   hipStream_t st = (hipStream_t)stream;
+  const bool one = Hh <= 32;  // (a last group of at most 32 heads beside full ones computes both tiles)
+#define SGL_ATTN(FMT)                                                   \
+  do {                                                                  \
+    if (one)                                                            \
+      sgl::sparse_attn_kernel<FMT, 1><<<grid, 512, 0, st>>>(a);         \
+    else                                                                \
+      sgl::sparse_attn_kernel<FMT, 2><<<grid, 512, 0, st>>>(a);         \
+  } while (0)
   if (kv_format == SGL_ATTN_KV_BF16)
-    sgl::sparse_attn_kernel<SGL_ATTN_KV_BF16><<<grid, 512, 0, st>>>(a);
+    SGL_ATTN(SGL_ATTN_KV_BF16);
   else if (kv_format == SGL_ATTN_KV_A)
-    sgl::sparse_attn_kernel<SGL_ATTN_KV_A><<<grid, 512, 0, st>>>(a);
+    SGL_ATTN(SGL_ATTN_KV_A);
   else
-    sgl::sparse_attn_kernel<SGL_ATTN_KV_A_PAGED><<<grid, 512, 0, st>>>(a);
+    SGL_ATTN(SGL_ATTN_KV_A_PAGED);
+#undef SGL_ATTN
   if (a.nsplit > 1) {
     const int64_t rows = B * M * Hh;
     sgl::sparse_attn_combine_kernel<<<(unsigned)sgl::ceil_div(rows, (int64_t)4), 256, 0, st>>>(a, rows);

@@ -67,12 +67,7 @@ __device__ __forceinline__ const uint8_t* uniform_ptr(const void* p) {
   return (const uint8_t*)(uintptr_t)(((uint64_t)hi << 32) | lo);
 }
 
-// Lane i of the wavefront copies 16 bytes from base + voff to LDS m0 + 16 i.
-__device__ __forceinline__ void dma16(const uint8_t* base, uint32_t voff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               :: "v"(voff), "s"(base), "s"(lds) : "memory");
-}
-// dma16 with the nontemporal cache policy: for operand bytes read once per
+// dma16 (sgl_common.h) with the nontemporal cache policy: for operand bytes read once per
 // launch (a nontemporal read stream on gfx950 moves 7.0 TB/s, a plain one 6.2)
 __device__ __forceinline__ void dma16nt(const uint8_t* base, uint32_t voff, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt"

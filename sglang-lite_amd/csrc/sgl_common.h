@@ -55,6 +55,13 @@ __device__ __forceinline__ uint32_t lds_u32(const void* p) {
   return (uint32_t)(uintptr_t)((__attribute__((address_space(3))) const uint8_t*)p);
 }
 
+// LDS DMA: lane i of the wavefront copies 16 bytes from base + voff to LDS m0 + 16 i
+// (global_load_lds_dwordx4; counted by vmcnt).
+__device__ __forceinline__ void dma16(const uint8_t* base, uint32_t voff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               :: "v"(voff), "s"(base), "s"(lds) : "memory");
+}
+
 // LDS DMA with a per-lane 64-bit address: lane i copies 16 bytes from addr to
 // LDS m0 + 16 i (global_load_lds_dwordx4; counted by vmcnt).
 __device__ __forceinline__ void dma16v(uint64_t addr, uint32_t lds) {

@@ -8,6 +8,8 @@ import pytest
 import torch
 
 from helpers import assert_gemm_close, bf16_values, f32, to_dev_bf16, to_dev_f32
+from oracle import attn as OA
+from oracle import kv as OK
 from oracle import moe as OM
 from test_gpu_fp4 import fp4_table
 from test_gpu_moe import table_from
@@ -35,3 +37,80 @@ def test_moe_tile_rule(gpu, fp4, T):
     table = (fp4_table if fp4 else table_from)(experts, sh, gpu)
     y = M.moe_forward(to_dev_bf16(x, gpu), torch.from_numpy(ids).to(gpu), to_dev_f32(w, gpu), table)
     assert_gemm_close(f32(y), OM.moe_forward(x, ids, w, experts, sh), f"tile rule T={T}")
+
+
+def _attn(gpu, q, kv, sink, idx, scale, fmt):
+    """(device output, the rows as the device reads them) for a bf16 cache,
+    packed rows or packed pages of 3 rows (not a power of two)."""
+    from sglang_lite_amd import dsv4_kv_pack as KVP
+    from sglang_lite_amd import v4_sparse_mla as SA
+
+    qd, kvd, sd = to_dev_bf16(q, gpu), to_dev_bf16(kv, gpu), to_dev_f32(sink, gpu)
+    idd = torch.from_numpy(idx).to(gpu)
+    if fmt == "bf16":
+        return f32(SA.sparse_attn(qd, kvd, sd, idd, scale)), kv
+    packed = KVP.pack_dsv4_kv_bf16(kvd)
+    rows = np.stack([OK.dequant_row_a(p.cpu().numpy()) for p in packed])
+    cache = packed if fmt == "rows" else torch.stack([KVP.to_paged_hnd(p, 3) for p in packed])
+    return f32(SA.sparse_attn_packed(qd, cache, sd, idd, scale, n_rows=kv.shape[1])), rows
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "rows", "pages"])
+@pytest.mark.parametrize("H", [1, 8, 32, 33, 64, 100])
+def test_sparse_attn_row_counts_at_block_edges(gpu, H, fmt):
+    """Valid rows per query at the edges of the 32-row blocks and of the tile
+    ring, masked entries between them, head counts at the edges of the
+    16- and 32-head tiles and of the 64-head groups."""
+    counts = [0, 1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 95, 96, 97, 128, 130]
+    rng = np.random.default_rng(H)
+    S, n, K = len(counts), 150, 160
+    print(f"attn edges H={H} {fmt}", flush=True)
+    q, kv = bf16_values(rng, (1, S, H, 512)), bf16_values(rng, (1, n, 512))
+    sink = (rng.standard_normal(H) * 2).astype(np.float32)
+    idx = np.full((1, S, K), -1, np.int32)
+    for s, c in enumerate(counts):
+        idx[0, s, np.sort(rng.permutation(K)[:c])] = rng.permutation(n)[:c]
+    got, rows = _attn(gpu, q, kv, sink, idx, 512 ** -0.5, fmt)
+    assert_gemm_close(got, OA.sparse_attn_blocked(q, rows, sink, idx, 512 ** -0.5), f"H={H} {fmt}")
+    assert np.all(got[0, 0] == 0)
+
+
+@pytest.mark.parametrize("fmt,K", [("bf16", 2752), ("bf16", 2753), ("rows", 1792), ("pages", 1793)])
+@pytest.mark.parametrize("queries", [1, 300])
+def test_sparse_attn_row_list_edges(gpu, fmt, K, queries):
+    """Selections that fill the row list of a workgroup exactly and by one more
+    (300 queries: unsplit; one: split, shorter lists)."""
+    rng = np.random.default_rng(K)
+    print(f"attn list K={K} queries={queries} {fmt}", flush=True)
+    q, kv = bf16_values(rng, (1, queries, 2, 512)), bf16_values(rng, (1, 40, 512))
+    sink = rng.standard_normal(2).astype(np.float32)
+    idx = rng.integers(0, 40, (1, queries, K)).astype(np.int32)
+    idx[0, :, ::7] = -1
+    got, rows = _attn(gpu, q, kv, sink, idx, 512 ** -0.5, fmt)
+    for s in (0, queries - 1):  # each query by itself: the oracle gathers every row
+        ref = OA.sparse_attn_exact(q[:, s:s + 1], rows, sink, idx[:, s:s + 1], 512 ** -0.5)
+        assert_gemm_close(got[:, s:s + 1], ref, f"K={K} query {s}")
+
+
+@pytest.mark.parametrize("order", ["rising", "falling", "one late"])
+def test_sparse_attn_moving_reference(gpu, order):
+    """Scores that rise block after block (the reference moves in each), fall,
+    or jump in the last block; and a row 0 that no query selects holding
+    infinities and NaN (the rows that pad a block read zeros, never it)."""
+    rng = np.random.default_rng(len(order))
+    n, K, H, S = 201, 200, 64, 260
+    q = np.zeros((1, S, H, 512), np.float32)
+    q[..., 0] = 8.0
+    q[..., 1:4] = bf16_values(rng, (1, S, H, 3))
+    kv = bf16_values(rng, (1, n, 512))
+    rank = {"rising": np.arange(K), "falling": np.arange(K)[::-1], "one late": (np.arange(K) == 199) * 150}
+    kv[0, 1:, 0] = np.float32(0.25) * np.floor(rank[order] * 0.5)  # scores up to 200 apart, exact in bf16
+    kv[0, 0] = np.array([np.inf, np.nan] * 256, np.float32)
+    idx = np.broadcast_to(np.arange(1, n, dtype=np.int32), (1, S, K)).copy()
+    sink = rng.standard_normal(H).astype(np.float32)
+    got, _ = _attn(gpu, q, kv, sink, idx, 1.0, "bf16")
+    ref = OA.sparse_attn_exact(q[:, :1], kv, sink, idx[:, :1], 1.0)
+    assert np.all(np.isfinite(got))
+    assert_gemm_close(got[:, :1], ref, order)
+    for s in (1, S - 1):
+        assert_gemm_close(got[:, s:s + 1], OA.sparse_attn_exact(q[:, s:s + 1], kv, sink, idx[:, s:s + 1], 1.0), order)
