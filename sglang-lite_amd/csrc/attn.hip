@@ -231,6 +231,7 @@ __device__ __forceinline__ void attn_role(const AttnArgs& a, Smem<FMT>& sm) {
   const int64_t k_begin = (int64_t)jb * kBlk;
   const int64_t k_end = min((int64_t)min(jb + a.bps, nblk_all) * kBlk, a.K);
 
+  int moves = 0;  // of the references
   bool first = true;
   for (int64_t kc = k_begin; kc < k_end || first; kc += kList<FMT>) {
     // ---- the chunk's valid rows, packed in order, padded to a whole block.
@@ -387,28 +388,35 @@ __device__ __forceinline__ void attn_role(const AttnArgs& a, Smem<FMT>& sm) {
     };
     // Block n has a score above its head's reference: the reference of a head
     // moves to its block maximum where that exceeds it by more than 8 (log2
-    // units): the probabilities stay <= 256 (exact range in bf16, same
-    // relative rounding).  Any reference gives the same softmax.  Both roles
-    // come here, the S wavefronts with block n's scores in st.
-    auto move_refs = [&](int n) {
-      if constexpr (S) {
-        if (live) {
+    // units; the second time by anything, since the largest probability, 1,
+    // is exact in bf16 and the first 32 rows hold it less often): the
+    // probabilities stay <= 256 (exact range in bf16, same relative rounding).
+    // Any reference gives the same softmax.  Both roles come here, the S
+    // wavefronts with block n's scores in st.
+    auto put_max = [&]() {
 #pragma unroll
-          for (int i = 0; i < 2; ++i) {
-            float mx = __builtin_fmaxf(__builtin_fmaxf(st[i][0], st[i][1]), __builtin_fmaxf(st[i][2], st[i][3]));
-            mx = __builtin_fmaxf(mx, __shfl_xor(mx, 16, 64));
-            mx = __builtin_fmaxf(mx, __shfl_xor(mx, 32, 64));
-            if (g4 == 0) sm.mx[th][32 * hh + 16 * i + l16] = mx;
-          }
-        }
+      for (int i = 0; i < 2; ++i) {
+        float mx = __builtin_fmaxf(__builtin_fmaxf(st[i][0], st[i][1]), __builtin_fmaxf(st[i][2], st[i][3]));
+        mx = __builtin_fmaxf(mx, __shfl_xor(mx, 16, 64));
+        mx = __builtin_fmaxf(mx, __shfl_xor(mx, 32, 64));
+        if (g4 == 0) sm.mx[th][32 * hh + 16 * i + l16] = mx;
       }
-      lds_barrier();  // maxima exchanged
+    };
+    auto move_refs = [&](int n) {
+      if (moves > 0) {  // (the first block leaves its maxima, and no P)
+        if constexpr (S) {
+          if (live) put_max();
+        }
+        lds_barrier();  // maxima exchanged
+      }
+      const float slack = moves < 2 ? 0.0f : 8.0f;
+      ++moves;
       float f[2];
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         const int h = S ? 32 * hh + 16 * i + l16 : 32 * i + c32;
         const float mx = __builtin_fmaxf(sm.mx[0][h], sm.mx[1][h]) * c1;  // (scale > 0)
-        const float mn = !(mx <= mref[i] + 8.0f) ? __builtin_fmaxf(mref[i], mx) : mref[i];
+        const float mn = !(mx <= mref[i] + slack) ? __builtin_fmaxf(mref[i], mx) : mref[i];
         f[i] = mn == mref[i] ? 1.0f : __builtin_amdgcn_exp2f(mref[i] - (mn == NEG_INF ? 0.0f : mn));
         mref[i] = mn;
       }
@@ -418,7 +426,7 @@ __device__ __forceinline__ void attn_role(const AttnArgs& a, Smem<FMT>& sm) {
           for (int i = 0; i < 2; ++i) {
             lsum[i] *= f[i];
             nref[i] = mref[i] == NEG_INF ? 0.0f : -mref[i];
-            lim[i] = (mref[i] + 8.0f) / c1;
+            lim[i] = (mref[i] + (moves < 2 ? 0.0f : 8.0f)) / c1;
           }
           put_p(n);
         }
@@ -480,13 +488,14 @@ __device__ __forceinline__ void attn_role(const AttnArgs& a, Smem<FMT>& sm) {
             for (int r = 0; r < 4; ++r)
               if (r >= left) st[0][r] = st[1][r] = NEG_INF;
           }
-          bool over = false;  // (also while the reference is -inf)
+          bool over = moves == 0;
 #pragma unroll
           for (int i = 0; i < 2; ++i)
             over |= !(__builtin_fmaxf(__builtin_fmaxf(st[i][0], st[i][1]),
                                       __builtin_fmaxf(st[i][2], st[i][3])) <= lim[i]);
           if (__ballot(over) && lane == 0) sm.flag[n & 3] = 1;
-          put_p(n);
+          if (moves == 0) put_max();
+          else put_p(n);
         }
         lds_barrier();
       }
