@@ -11,6 +11,7 @@
 #include <mutex>
 
 #include "sgl_gemm.h"
+#include "sgl_moe_small.h"
 #include "sgl_numeric.h"
 
 namespace sgl {
@@ -1300,6 +1301,27 @@ int sgl_moe_forward(const void* x, int64_t T, int64_t H, int64_t I, int E, int k
   if ((rc = sgl_act_quant(x, T, H, H, w.xq, H, w.xs, H / 128, 128, scale_mode, 0, 0, stream)))
     return rc;
   hipStream_t st = (hipStream_t)stream;
+  const bool fp4 = sgl::fp4_experts(expert_format);
+  if (sgl::small_moe_ok(T, H, I, k, has_shared, fp4)) {
+    sgl::SmallMoeArgs a = {};
+    a.xq = w.xq;
+    a.xs = w.xs;
+    a.ids = ids;
+    a.route_w = weights;
+    a.experts = experts;
+    a.T = T;
+    a.H = H;
+    a.I = I;
+    a.E = E;
+    a.k = k;
+    a.has_shared = has_shared;
+    a.swiglu_limit = swiglu_limit;
+    a.scale_mode = scale_mode;
+    a.sa_pow2 = sgl::pow2_scale_mode(scale_mode);
+    a.h = w.out;  // [T (k + shared), I] in the rows [T (k + shared), H] of the grouped path
+    a.y = (uint16_t*)y;
+    return sgl::launch_small_moe(a, fp4, st);
+  }
   // the permute also zeroes the GEMMs' tile counters
   if ((rc = sgl::launch_permute(ids, T, k, E, w.counts, w.offsets, w.sorted_slot, w.slot_pos,
                                 w.tile_ctr, sgl::kTileCtrs, st)))

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import assert_gemm_close, bf16_values, f32, to_dev_bf16, to_dev_f32
+from helpers import assert_gemm_close, assert_layer_close, bf16_values, f32, to_dev_bf16, to_dev_f32
 from oracle import attn as OA
 from oracle import kv as OK
 from oracle import moe as OM
@@ -37,6 +37,48 @@ def test_moe_tile_rule(gpu, fp4, T):
     table = (fp4_table if fp4 else table_from)(experts, sh, gpu)
     y = M.moe_forward(to_dev_bf16(x, gpu), torch.from_numpy(ids).to(gpu), to_dev_f32(w, gpu), table)
     assert_gemm_close(f32(y), OM.moe_forward(x, ids, w, experts, sh), f"tile rule T={T}")
+
+
+@pytest.mark.parametrize("fp4,T,H,I,E,k,shared,mode", [
+    (False, 1, 4096, 2048, 12, 8, True, 0),
+    (False, 1, 4224, 384, 20, 16, False, 2),   # 33 K lines, 16 slots, no shared expert
+    (False, 2, 512, 512, 4, 4, True, 3),       # 8 slots; power-of-two scales
+    (False, 2, 640, 512, 6, 5, True, 0),       # 10 slots: the grouped path
+    (False, 1, 256, 384, 4, 2, True, 0),       # I > H: the grouped path
+    (True, 1, 4096, 2048, 10, 8, True, 3),
+    (True, 1, 512, 256, 3, 1, True, 0),        # fewer K lines than wavefronts
+    (True, 3, 2560, 2304, 9, 8, True, 1),      # 24 slots, I past 16 lines
+    (True, 4, 512, 512, 7, 6, False, 2),       # 24 slots, no shared expert
+    (True, 12, 512, 512, 5, 2, True, 3),       # 24 slots, rows of the shared expert 12
+    (True, 24, 512, 512, 5, 1, True, 0),       # two 16-row tiles of the shared expert
+    (True, 5, 512, 512, 7, 5, True, 3),        # 25 slots: the grouped path
+])
+def test_moe_smallest_batches(gpu, fp4, T, H, I, E, k, shared, mode):
+    """The layer of one to a few tokens and the sizes where it gives way to
+    the grouped path; an id outside the experts adds nothing, and a token may
+    name an expert twice (the oracle: the same slot with weight 0, and a copy
+    of that expert under an id of its own)."""
+    from sglang_lite_amd import moe as M
+
+    rng = np.random.default_rng(T * 1000 + H + I + mode)
+    print(f"smallest fp4={fp4} T={T} H={H} I={I} E={E} k={k} shared={shared} mode={mode}", flush=True)
+    x = bf16_values(rng, (T, H))
+    ids = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.int32)
+    w = rng.uniform(0.1, 1.0, (T, k)).astype(np.float32)
+    dev_ids, ref_w = ids.copy(), w.copy()
+    if T * k > 8:
+        dev_ids[0, k - 1], ref_w[0, k - 1] = (-1 if T % 2 else E), 0.0
+    if k > 2:
+        dev_ids[T - 1, 1], ids[T - 1, 1] = ids[T - 1, 0], E
+    ue = mode in (1, 3)
+    experts = [OM.make_fp4_expert(rng, H, I) if fp4 else OM.make_expert(rng, H, I, ue8m0=ue) for _ in range(E)]
+    sh = OM.make_expert(rng, H, I, ue8m0=ue) if shared else None
+    table = (fp4_table if fp4 else table_from)(experts, sh, gpu)
+    y = M.moe_forward(to_dev_bf16(x, gpu), torch.from_numpy(dev_ids).to(gpu), to_dev_f32(w, gpu), table,
+                      swiglu_limit=3.0, scale_mode=mode)
+    experts = experts + [experts[ids[T - 1, 0]]]
+    y_ref = OM.moe_forward(x, ids, ref_w, experts, sh, swiglu_limit=3.0, mode=mode)
+    assert_layer_close(f32(y), y_ref, f"smallest T={T} k={k}")
 
 
 def _attn(gpu, q, kv, sink, idx, scale, fmt):
