@@ -81,6 +81,49 @@ def test_moe_smallest_batches(gpu, fp4, T, H, I, E, k, shared, mode):
     assert_layer_close(f32(y), y_ref, f"smallest T={T} k={k}")
 
 
+@pytest.mark.parametrize("scales", ["fp32", "e8m0", "mixed"])
+@pytest.mark.parametrize("M,N,K", [
+    (17, 208, 128),     # one K block (three of a stage's four groups idle), a ragged column tile
+    (33, 1040, 640),    # five K blocks: a last stage of one
+    (64, 1600, 256),    # split-K shape that the K groups take; two K blocks
+    (32, 512, 4096),    # split-K shape that stays split
+    (130, 2048, 896),   # 5 x 32 tiles of 32 x 64, seven K blocks
+    (257, 2048, 384),   # past one round of 32 x 64: 32 x 128, an odd K block at the end
+    (513, 2048, 7168),  # past one round of 32 x 128: 64 x 128, the longest K its scale table holds
+    (500, 2048, 7296),  # one K block more: the tiles before
+    (200, 512, 8192),   # the longest K of the 32-row tiles' scale table
+    (200, 512, 8320),
+    (2060, 1536, 256),  # few 256 x 256 tiles: several rounds of 64 x 128
+])
+def test_fp8_gemm_k_groups(gpu, M, N, K, scales):
+    """The dense product on both sides of each tile rule against the
+    dequantized product, in both output types."""
+    from sglang_lite_amd import kernel as KK
+    from sglang_lite_amd import v4_deep_gemm as DG
+
+    print(f"k groups M={M} N={N} K={K} {scales}", flush=True)
+    gen = torch.Generator(device=gpu).manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=gen, device=gpu).bfloat16()
+    b = (torch.randn(N, K, generator=gen, device=gpu) * 90).clamp_(-448, 448).to(torch.float8_e4m3fn)
+    nb = (N + 127) // 128
+    if scales == "fp32":
+        a, sa = KK.act_quant(x, 128)
+        sb = torch.rand(nb, K // 128, generator=gen, device=gpu) * 1e-4 + 1e-4
+    else:
+        a, sa = KK.act_quant(x, 128, "ue8m0", torch.float8_e8m0fnu)
+        sb = torch.randint(110, 118, (nb, K // 128), generator=gen, device=gpu, dtype=torch.uint8).view(
+            torch.float8_e8m0fnu)
+        if scales == "mixed":
+            sb = sb.float()
+    ad = a.double() * sa.float().double().repeat_interleave(128, 1)
+    bd = b.double() * sb.float().double().repeat_interleave(128, 0)[:N].repeat_interleave(128, 1)
+    ref = (ad @ bd.t().contiguous()).float().cpu().numpy()
+    for dt in (torch.bfloat16, torch.float32):
+        c = DG.fp8_gemm_nt(a, sa, b, sb, out_dtype=dt)
+        assert c.dtype == dt
+        assert_gemm_close(f32(c) if dt == torch.bfloat16 else c.cpu().numpy(), ref, f"{M}x{N}x{K} {scales} {dt}")
+
+
 def _attn(gpu, q, kv, sink, idx, scale, fmt):
     """(device output, the rows as the device reads them) for a bf16 cache,
     packed rows or packed pages of 3 rows (not a power of two)."""
