@@ -8,6 +8,7 @@ missing or a call fails, the caller gets an exception.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from ctypes import c_float, c_int, c_int64, c_size_t, c_void_p
 from pathlib import Path
@@ -115,6 +116,8 @@ SIGNATURES = {
 }
 
 _LIB: Optional[ctypes.CDLL] = None
+_FN: dict = {}         # the bound functions of _LIB by name
+_RAW_STREAM = None     # torch's raw current-stream getter, by device index
 
 
 class SglError(RuntimeError):
@@ -159,6 +162,7 @@ def load(path: Optional[os.PathLike] = None) -> ctypes.CDLL:
     if ver != ABI_VERSION:
         raise RuntimeError(f"sglang_lite_amd: ABI version {ver}, expected {ABI_VERSION}")
     if path is None:
+        _FN.clear()
         _LIB = lib
     return lib
 
@@ -181,8 +185,24 @@ def check(status: int, what: str) -> None:
 
 
 def call(name: str, *args) -> None:
-    fn = getattr(load(), name)
-    check(fn(*args), name)
+    fn = _FN.get(name) if _LIB is not None else None
+    if fn is None:
+        fn = getattr(load(), name)
+        _FN[name] = fn
+    status = fn(*args)
+    if status != SGL_OK:
+        check(status, name)
+
+
+@functools.lru_cache(maxsize=1024)
+def _size(lib, name: str, args: tuple) -> int:
+    return int(getattr(lib, name)(*args))
+
+
+def size_of(name: str, *args: int) -> int:
+    """A ``sgl_*_workspace_size`` function: pure functions of the sizes, asked
+    on every call of their operation, so the last answers are kept."""
+    return _size(load(), name, args)
 
 
 def ptr(t) -> Optional[int]:
@@ -192,9 +212,14 @@ def ptr(t) -> Optional[int]:
 
 def stream_of(t) -> int:
     """HIP stream handle torch is currently using on ``t``'s device."""
-    import torch
+    global _RAW_STREAM
+    if _RAW_STREAM is None:
+        import torch
 
-    return torch.cuda.current_stream(t.device).cuda_stream
+        # the handle alone, without the Stream object torch.cuda.current_stream makes (1.5 us a call)
+        _RAW_STREAM = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+            lambda index: torch.cuda.current_stream(index).cuda_stream)
+    return _RAW_STREAM(t.get_device())
 
 
 def require_device(*tensors, what: str) -> None:

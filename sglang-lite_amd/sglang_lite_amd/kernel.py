@@ -36,7 +36,10 @@ FUSED_ACT_QUANT = "_sglang_lite_amd_act_quant"
 
 
 def act_quant_formula() -> str:
-    raw = os.environ.get("SGLANG_LITE_AMD_ACT_QUANT", "torch").strip().lower()
+    raw = os.environ.get("SGLANG_LITE_AMD_ACT_QUANT")
+    if raw is None:
+        return "torch"
+    raw = raw.strip().lower()
     if raw not in ("torch", "tilelang"):
         raise ValueError(f"SGLANG_LITE_AMD_ACT_QUANT must be 'torch' or 'tilelang', got {raw!r}")
     return raw
@@ -184,6 +187,12 @@ def fp8_gemm(
     (bf16 or fp32).  ``scale_dtype`` is accepted for signature parity; the
     scale tensors' own dtypes (fp32 or e8m0) decide how they are read."""
     del scale_dtype
+    return fp8_gemm_as(a, a_s, b, b_s, torch.get_default_dtype(), out)
+
+
+def fp8_gemm_as(a: torch.Tensor, a_s: torch.Tensor, b: torch.Tensor, b_s: torch.Tensor,
+                odt: torch.dtype, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """:func:`fp8_gemm` with the output dtype given."""
     assert a.is_contiguous() and b.is_contiguous(), "Input tensors must be contiguous"
     assert a_s.is_contiguous() and b_s.is_contiguous(), "Scaling factor tensors must be contiguous"
     _lib.require_device(a, a_s, b, b_s, what="fp8_gemm")
@@ -192,7 +201,6 @@ def fp8_gemm(
     K = a.size(-1)
     M = a.numel() // K
     N = b.size(0)
-    odt = torch.get_default_dtype()
     if odt not in (torch.bfloat16, torch.float32):
         raise TypeError(f"fp8_gemm: default dtype must be bfloat16 or float32, got {odt}")
     if out is None:
@@ -202,7 +210,7 @@ def fp8_gemm(
     # split-K shapes keep their fp32 partials in a workspace allocated here with
     # torch (inside a graph capture it comes from the graph's pool), as the
     # reference's adapter allocates its output (engine/v4_deep_gemm.py:186-188)
-    nws = int(_lib.load().sgl_fp8_gemm_workspace_size(M, N, K)) if M else 0
+    nws = _lib.size_of("sgl_fp8_gemm_workspace_size", M, N, K) if M else 0
     ws = torch.empty(nws, dtype=torch.uint8, device=a.device) if nws else None
     _lib.call(
         "sgl_fp8_gemm",
@@ -250,6 +258,13 @@ def fp4_gemm(
     scales are applied inside the MFMA; otherwise each 128-deep partial is
     promoted with the fp32 activation scale.  K % 256 == 0."""
     del scale_dtype
+    return fp4_gemm_as(a, a_s, b, b_s, torch.get_default_dtype(), out, a_scale_pow2)
+
+
+def fp4_gemm_as(a: torch.Tensor, a_s: torch.Tensor, b: torch.Tensor, b_s: torch.Tensor,
+                odt: torch.dtype, out: Optional[torch.Tensor] = None,
+                a_scale_pow2: Optional[bool] = None) -> torch.Tensor:
+    """:func:`fp4_gemm` with the output dtype given."""
     assert a.is_contiguous() and b.is_contiguous(), "Input tensors must be contiguous"
     assert a_s.is_contiguous() and b_s.is_contiguous(), "Scaling factor tensors must be contiguous"
     _lib.require_device(a, a_s, b, b_s, what="fp4_gemm")
@@ -261,7 +276,6 @@ def fp4_gemm(
     N = b.size(0)
     if bq.dim() != 2 or bq.size(1) * 2 != K:
         raise ValueError(f"fp4_gemm: weight must be [N, K/2] = [{N}, {K // 2}], got {tuple(b.shape)}")
-    odt = torch.get_default_dtype()
     if odt not in (torch.bfloat16, torch.float32):
         raise TypeError(f"fp4_gemm: default dtype must be bfloat16 or float32, got {odt}")
     if out is None:

@@ -334,8 +334,7 @@ def moe_forward(x: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, table
     k = ids.shape[1]
     if H != table.H:
         raise ValueError(f"moe_forward: x has H={H}, experts have H={table.H}")
-    lib = _lib.load()
-    nbytes = int(lib.sgl_moe_workspace_size(T, H, table.I, table.E, k, int(table.has_shared)))
+    nbytes = workspace_size(T, H, table.I, table.E, k, table.has_shared)
     ws = (workspace or MoEWorkspace()).get(nbytes, x.device)
     y = out if out is not None else torch.empty(T, H, dtype=torch.bfloat16, device=x.device)
     _lib.call("sgl_moe_forward", x.data_ptr(), T, H, table.I, table.E, k, ids.data_ptr(),
@@ -394,7 +393,7 @@ def moe_add_shared(y_local: torch.Tensor, table: ExpertTable, k: int,
 
 
 def workspace_size(T: int, H: int, I: int, E: int, k: int, has_shared: bool) -> int:
-    return int(_lib.load().sgl_moe_workspace_size(T, H, I, E, k, int(has_shared)))
+    return _lib.size_of("sgl_moe_workspace_size", T, H, I, E, k, int(has_shared))
 
 
 __all__ = ["ExpertTable", "MoEWorkspace", "combine", "down", "gate", "gate_up", "moe_add_shared",

@@ -162,10 +162,10 @@ def fp8_gemm_nt(a: torch.Tensor, a_s: torch.Tensor, b: torch.Tensor, b_s: torch.
     M = a.numel() // K
     N = b.size(0)
     odt = out_dtype or torch.get_default_dtype()
-    a2 = a.reshape(M, K)
+    a2 = a if a.dim() == 2 else a.reshape(M, K)
     if not a2.is_contiguous():
         a2 = a2.contiguous()
-    as2 = a_s.reshape(M, -1)
+    as2 = a_s if a_s.dim() == 2 and a_s.size(0) == M else a_s.reshape(M, -1)
     if not as2.is_contiguous():
         as2 = as2.contiguous()
     if getattr(b, "_dg_s_f32", None) is not None:
@@ -176,13 +176,9 @@ def fp8_gemm_nt(a: torch.Tensor, a_s: torch.Tensor, b: torch.Tensor, b_s: torch.
         bs = b_s.contiguous()
     bb = b if b.is_contiguous() else b.contiguous()
     res = out if out is not None and out.dtype == odt and out.is_contiguous() else None
-    prev = torch.get_default_dtype()
-    try:
-        torch.set_default_dtype(odt)
-        c = HK.fp8_gemm(a2, as2, bb, bs, out=res.view(M, N) if res is not None else None)
-    finally:
-        torch.set_default_dtype(prev)
-    c = c.view(*a.shape[:-1], N)
+    c = HK.fp8_gemm_as(a2, as2, bb, bs, odt, res.view(M, N) if res is not None else None)
+    if a.dim() != 2:
+        c = c.view(*a.shape[:-1], N)
     if out is not None and res is None:
         out.copy_(c)
         return out
@@ -201,10 +197,10 @@ def fp4_gemm_nt(a: torch.Tensor, a_s: torch.Tensor, b: torch.Tensor, b_s: torch.
     M = a.numel() // K
     N = b.size(0)
     odt = out_dtype or torch.get_default_dtype()
-    a2 = a.reshape(M, K)
+    a2 = a if a.dim() == 2 else a.reshape(M, K)
     if not a2.is_contiguous():
         a2 = a2.contiguous()
-    as2 = a_s.reshape(M, -1)
+    as2 = a_s if a_s.dim() == 2 and a_s.size(0) == M else a_s.reshape(M, -1)
     if not as2.is_contiguous():
         as2 = as2.contiguous()
     if getattr(b, "_sgl_w_u8", None) is not None and getattr(b, "_sgl_s_e8m0", None) is not None:
@@ -215,13 +211,9 @@ def fp4_gemm_nt(a: torch.Tensor, a_s: torch.Tensor, b: torch.Tensor, b_s: torch.
         bi = HK.fp4_bytes(b if b.is_contiguous() else b.contiguous())
         bs = HK.fp4_weight_scale(b_s)
     res = out if out is not None and out.dtype == odt and out.is_contiguous() else None
-    prev = torch.get_default_dtype()
-    try:
-        torch.set_default_dtype(odt)
-        c = HK.fp4_gemm(a2, as2, bi, bs, out=res.view(M, N) if res is not None else None)
-    finally:
-        torch.set_default_dtype(prev)
-    c = c.view(*a.shape[:-1], N)
+    c = HK.fp4_gemm_as(a2, as2, bi, bs, odt, res.view(M, N) if res is not None else None)
+    if a.dim() != 2:
+        c = c.view(*a.shape[:-1], N)
     if out is not None and res is None:
         out.copy_(c)
         return out

@@ -64,7 +64,7 @@ def _launch(q, kv, fmt, page, n, bstride, ld, attn_sink, topk_idxs, softmax_scal
     sink = attn_sink.to(torch.float32).contiguous()
     o = torch.empty_like(qc)
     k = idx.shape[-1]
-    ws_bytes = int(_lib.load().sgl_sparse_attn_workspace_size(b, s, h, k)) if k > 0 else 0
+    ws_bytes = _lib.size_of("sgl_sparse_attn_workspace_size", b, s, h, k) if k > 0 else 0
     ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=qc.device)
     _lib.call("sgl_sparse_attn", qc.data_ptr(), b, s, h, kv.data_ptr(), fmt, page, n, bstride, ld,
               sink.data_ptr(), idx.data_ptr(), k, float(softmax_scale), o.data_ptr(),
