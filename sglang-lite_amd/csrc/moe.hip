@@ -292,8 +292,10 @@ __global__ __launch_bounds__(64 * NWV) void router_logits_kernel(const uint16_t*
 // Router projection for prefill-sized batches (H % 64 == 0).  A workgroup
 // of four wavefronts owns TT tokens x TE experts; the x and W rows stream
 // through an NS-deep ring of 64-deep LDS stages (TT + TE rows of 128 bytes)
-// by global_load_lds_dwordx4, one instruction filling 8 rows x 128 bytes, the
-// 16-byte chunks swizzled (chunk c of row r at c ^ swz(r)), NS - 1 stages in
+// by global_load_lds_dwordx4 (G > 1: G such groups of four wavefronts, each with
+// a 64-deep K block of the stage of its own, their partial tiles summed in
+// order through LDS), one instruction filling 8 rows x 128 bytes, the 16-byte
+// chunks swizzled (chunk c of row r at c ^ swz(r)), NS - 1 stages in
 // flight.  Whole 128-byte row segments per instruction are what the L2 serves
 // fastest; the register-loaded kernel above reads 16 rows x 64 bytes per
 // instruction.  A wavefront computes a (TT/WT) x (TE/WE) block with
@@ -317,8 +319,8 @@ __device__ __forceinline__ void router_wait(int later) {
   }
 }
 
-template <int TT, int TE, int NS>
-__global__ __launch_bounds__(256) void router_lds_kernel(const uint16_t* __restrict__ x,
+template <int TT, int TE, int NS, int G>
+__global__ __launch_bounds__(256 * G) void router_lds_kernel(const uint16_t* __restrict__ x,
                                                          const uint16_t* __restrict__ w, int64_t T,
                                                          int H, int E, int ntile_e, int64_t ntiles,
                                                          int64_t per_xcd, float* __restrict__ logits) {
@@ -328,16 +330,19 @@ __global__ __launch_bounds__(256) void router_lds_kernel(const uint16_t* __restr
   constexpr int ROWS = TT + TE;
   constexpr int SBYTES = ROWS * 128;
   constexpr int NI = ROWS / 32;  // DMA instructions per wavefront per stage
+  constexpr int STAGE = G * SBYTES;
   static_assert(ROWS % 32 == 0 && TT % 8 == 0 && ST % 16 == 0 && SE % 16 == 0, "tile shape");
   static_assert(NS >= 2 && (NS - 2) * NI <= 63, "vmcnt range");
-  __shared__ __align__(16) uint8_t ring[NS * SBYTES];
+  static_assert(NS * STAGE <= 160 * 1024 && (G == 1 || G * TT * TE * 4 <= NS * STAGE), "LDS");
+  __shared__ __align__(16) uint8_t ring[NS * STAGE];
 
   const int64_t tile = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   if (tile >= ntiles) return;
   const int64_t t0 = (tile / ntile_e) * TT;
   const int e0 = (int)(tile % ntile_e) * TE;
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);  // its K block of a stage
+  const int wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
 
   // instruction j of this wavefront fills stage rows 8 (wave + 4 j) + lane / 8
   uint64_t src[NI];
@@ -356,12 +361,14 @@ __global__ __launch_bounds__(256) void router_lds_kernel(const uint16_t* __restr
     src[j] = (uint64_t)(uintptr_t)row + 16u * (uint32_t)c;
   }
   const uint32_t ring0 = __builtin_amdgcn_readfirstlane(lds_u32(ring));
-  const int nst = H / 64;
+  const int nkb = H / 64, nst = (nkb + G - 1) / G;
   auto issue = [&](int s) {
-    const uint32_t slot = ring0 + (uint32_t)(s % NS) * SBYTES;
+    const int kb = s * G + grp;
+    if (G > 1 && kb >= nkb) return;
+    const uint32_t slot = ring0 + (uint32_t)(s % NS) * STAGE + (uint32_t)grp * SBYTES;
 #pragma unroll
     for (int j = 0; j < NI; ++j)
-      dma16v(src[j] + (uint64_t)s * 128u,
+      dma16v(src[j] + (uint64_t)kb * 128u,
              __builtin_amdgcn_readfirstlane(slot + (uint32_t)(8 * (wave + 4 * j)) * 128u));
   };
   for (int s = 0; s < NS - 1 && s < nst; ++s) issue(s);
@@ -376,12 +383,15 @@ __global__ __launch_bounds__(256) void router_lds_kernel(const uint16_t* __restr
 #pragma unroll
     for (int nj = 0; nj < NB; ++nj) acc[mi][nj] = v4f_r{0.0f, 0.0f, 0.0f, 0.0f};
   for (int s = 0; s < nst; ++s) {
-    // stage s has landed once at most min(NS - 2, nst - 1 - s) later stages are outstanding
-    const int later = nst - 1 - s < NS - 2 ? nst - 1 - s : NS - 2;
+    // stage s has landed once at most min(NS - 2, nst - 1 - s) later stages are
+    // outstanding (a group without a block in the last one waits for all before)
+    const int left = nst - 1 - s;
+    const int later = left >= NS - 1 || (G == 1 && left >= NS - 2) ? NS - 2 : (G == 1 ? left : 0);
     router_wait<NI, NS - 2>(later);
     __builtin_amdgcn_s_barrier();
     if (s + NS - 1 < nst) issue(s + NS - 1);
-    const uint8_t* st = ring + (s % NS) * SBYTES;
+    if (G > 1 && s * G + grp >= nkb) continue;
+    const uint8_t* st = ring + (s % NS) * STAGE + grp * SBYTES;
     v8bf alo[MB], ahi[MB], blo[NB], bhi[NB];
 #pragma unroll
     for (int mi = 0; mi < MB; ++mi) {
@@ -402,6 +412,28 @@ __global__ __launch_bounds__(256) void router_lds_kernel(const uint16_t* __restr
         acc[mi][nj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(alo[mi], blo[nj], acc[mi][nj], 0, 0, 0);
         acc[mi][nj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ahi[mi], bhi[nj], acc[mi][nj], 0, 0, 0);
       }
+  }
+  if constexpr (G > 1) {
+    // the groups' partial tiles meet in LDS and are summed in order
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    float* part = reinterpret_cast<float*>(ring);
+    auto at = [&](int row, int col) -> int { return row * TE + ((col + 16 * (row >> 2)) & (TE - 1)); };
+#pragma unroll
+    for (int mi = 0; mi < MB; ++mi)
+#pragma unroll
+      for (int nj = 0; nj < NB; ++nj)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          part[grp * TT * TE + at(wt * ST + 16 * mi + 4 * g4 + r, we * SE + 16 * nj + r16)] = acc[mi][nj][r];
+    __syncthreads();
+    for (int i = threadIdx.x; i < TT * TE; i += 256 * G) {
+      const int row = i / TE, col = i % TE;
+      float v = part[at(row, col)];
+#pragma unroll
+      for (int q = 1; q < G; ++q) v += part[q * TT * TE + at(row, col)];
+      if (t0 + row < T && e0 + col < E) logits[(t0 + row) * E + e0 + col] = v;
+    }
+    return;
   }
   // lane (g4, r16) holds tokens 4 g4 + r, expert r16 of each 16 x 16 block
 #pragma unroll
@@ -535,14 +567,14 @@ void launch_router_ks(const uint16_t* x, const uint16_t* w, int64_t T, int H, in
                                                                          per_xcd, logits);
 }
 
-template <int TT, int TE, int NS>
+template <int TT, int TE, int NS, int G = 1>
 void launch_router_lds(const uint16_t* x, const uint16_t* w, int64_t T, int H, int E,
                        float* logits, hipStream_t st) {
   const int ntile_e = (int)ceil_div(E, TE);
   const int64_t ntiles = ceil_div(T, TT) * ntile_e;
   const int64_t per_xcd = ceil_div(ntiles, 8);
-  router_lds_kernel<TT, TE, NS><<<(unsigned)(8 * per_xcd), 256, 0, st>>>(x, w, T, H, E, ntile_e, ntiles,
-                                                                          per_xcd, logits);
+  router_lds_kernel<TT, TE, NS, G><<<(unsigned)(8 * per_xcd), 256 * G, 0, st>>>(x, w, T, H, E, ntile_e, ntiles,
+                                                                                 per_xcd, logits);
 }
 
 // -------------------------------------------------------------- permute
@@ -1182,27 +1214,32 @@ int sgl_moe_gate(const void* x, const void* w, int64_t T, int64_t H, int E, int 
   const uint16_t* xb = (const uint16_t*)x;
   const uint16_t* wb = (const uint16_t*)w;
   // T > 256 with H % 64 == 0: the LDS-staged kernels, the largest of their
-  // tiles that still gives about a workgroup per CU; K split over the four
-  // wavefronts for the 32 x 64 and 32 x 32 tiles when H % 128 == 0 (H = 4096,
-  // E = 256 projection: T = 512 13.0 -> 9.4 us, T = 2048 18.3 -> 15.0 us; for
-  // 32 x 128 even, for 64 x 128 31.4 -> 33.6 us, so those keep 2 x 2
-  // wavefronts over 64-deep stages).  Decode-sized batches: the
-  // register-loaded kernel with 16 tokens x 16 experts per workgroup and 16
-  // wavefronts with all their K steps in flight (many small workgroups spread
-  // the weight read); it also serves H % 64 != 0 (64 x 64 or 64 x 128 tiles).
+  // tiles that still gives about a workgroup per CU.  K split over the four
+  // wavefronts for the 32 x 32 tiles when H % 128 == 0 (H = 4096, E = 256
+  // projection: T = 512 13.0 -> 9.4 us); for the larger tiles two or four
+  // groups of four wavefronts, a 64-deep K block of the stage each, as the
+  // serial chain of a stage is walked half or a quarter as often (gate, one
+  // group or the four-way split / these: T = 2048 19.8 / 18.5 us, 3000 31.2 /
+  // 28.4, 3900 29.6 / 27.9, 4200 36.9 / 32.5, 8192 43.4 / 43.0 on a repeated
+  // x and 40.5 / 36.2 on a fresh one, 16384 87.6 / 89.7; H = 7168: T = 5000
+  // 80 / 58, 16384 122.3 / 121.7).  The choice between them is one round of
+  // tiles where there is one (T = 6000 in two rounds of 32 x 128 46 us, in one
+  // of 64 x 128 34; T = 3000 27.1 in 32 x 128 tiles, but two sums as long
+  // instead of four err by 2.7e-7 rather than 1.9e-7).  Decode-sized
+  // batches: the register-loaded kernel with 16 tokens x 16 experts per
+  // workgroup and 16 wavefronts with all their K steps in flight (many small
+  // workgroups spread the weight read); it also serves H % 64 != 0 (64 x 64 or
+  // 64 x 128 tiles).
   auto tiles = [&](int64_t tt, int64_t te) { return sgl::ceil_div(T, tt) * sgl::ceil_div(E, te); };
-  if (T > 256 && H % 128 == 0 && tiles(32, 128) < 240) {
-    if (tiles(32, 64) >= 240)
-      sgl::launch_router_ks<32, 64, 6>(xb, wb, T, (int)H, E, logits, st);
-    else
-      sgl::launch_router_ks<32, 32, 8>(xb, wb, T, (int)H, E, logits, st);
+  if (T > 256 && H % 128 == 0 && tiles(32, 64) < 240) {
+    sgl::launch_router_ks<32, 32, 8>(xb, wb, T, (int)H, E, logits, st);
   } else if (T > 256 && H % 64 == 0) {
-    if (tiles(64, 128) >= 240)
-      sgl::launch_router_lds<64, 128, 4>(xb, wb, T, (int)H, E, logits, st);
+    if (tiles(32, 128) > 256)
+      sgl::launch_router_lds<64, 128, 3, 2>(xb, wb, T, (int)H, E, logits, st);
     else if (tiles(32, 128) >= 240)
-      sgl::launch_router_lds<32, 128, 4>(xb, wb, T, (int)H, E, logits, st);
+      sgl::launch_router_lds<32, 128, 3, 2>(xb, wb, T, (int)H, E, logits, st);
     else if (tiles(32, 64) >= 240)
-      sgl::launch_router_lds<32, 64, 6>(xb, wb, T, (int)H, E, logits, st);
+      sgl::launch_router_lds<32, 64, 3, 4>(xb, wb, T, (int)H, E, logits, st);
     else
       sgl::launch_router_lds<32, 32, 8>(xb, wb, T, (int)H, E, logits, st);
   } else if (T <= 256) {

@@ -199,3 +199,30 @@ def test_sparse_attn_moving_reference(gpu, order):
     assert_gemm_close(got[:, :1], ref, order)
     for s in (1, S - 1):
         assert_gemm_close(got[:, s:s + 1], OA.sparse_attn_exact(q[:, s:s + 1], kv, sink, idx[:, s:s + 1], 1.0), order)
+
+
+@pytest.mark.parametrize("T,H,E", [
+    (4096, 448, 256),   # 32 x 128 tiles in exactly one round; 7 K blocks for two groups
+    (4097, 64, 256),    # 64 x 128 tiles, one row past that round; the second group has no K block
+    (4110, 192, 250),   # ragged last tiles of both sides, 3 K blocks
+    (1921, 320, 256),   # 32 x 64 tiles, 5 K blocks for four groups
+    (2049, 64, 248),    # 32 x 64 tiles, one K block: three groups have none
+    (1920, 384, 256),   # 32 x 64 tiles from here (240), 6 K blocks
+    (1919, 384, 192),   # the four-way split's 32 x 32 tiles
+])
+def test_router_k_groups(gpu, T, H, E):
+    """The projection at the edges of its tile rule and with K blocks that the
+    groups share unevenly, within the fp32 summation bound of the exact logits:
+    H products summed in at most H additions of partial sums no larger than the
+    sum of magnitudes, in practice well below 2^-21 of it."""
+    from sglang_lite_amd import moe as M
+
+    print(f"router k groups T={T} H={H} E={E}", flush=True)
+    rng = np.random.default_rng(T + H + E)
+    x = bf16_values(rng, (T, H))
+    W = bf16_values(rng, (E, H))
+    lg = torch.full((T, E), float("nan"), dtype=torch.float32, device=gpu)
+    M.gate(to_dev_bf16(x, gpu), to_dev_bf16(W, gpu), 4, "sigmoid", None, 1.0, logits=lg)
+    exact = x.astype(np.float64) @ W.astype(np.float64).T
+    mag = np.abs(x).astype(np.float64) @ np.abs(W).astype(np.float64).T
+    assert np.all(np.abs(f32(lg).astype(np.float64) - exact) <= 2.0 ** -21 * mag + 1e-30)
