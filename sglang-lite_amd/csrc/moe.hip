@@ -685,76 +685,95 @@ __global__ __launch_bounds__(kPermThreads) void permute_kernel(const int32_t* __
   rank_slots(ids, 0, P, E, elo, ehi, run, wcnt, sorted_slot, slot_pos);
 }
 
-// Large inputs: chunks of kPermChunk slots, one workgroup each, in four
-// launches.  The per-chunk tables live in the outputs before the outputs are
-// final: (1) chunk histograms -> slot_pos[c*E + e]; (2) one workgroup sums
-// them into counts / offsets and writes each chunk's start position per
-// expert -> sorted_slot[c*E + e]; (3) each chunk ranks its slots from those
-// starts and writes slot_pos; (4) sorted_slot[slot_pos[i]] = i.  Needs
-// chunks * E <= P (checked by the caller).
-constexpr int kPermChunk = 4096;
-
-__global__ __launch_bounds__(kPermThreads) void permute_hist_kernel(const int32_t* __restrict__ ids,
-                                                                    int64_t P, int E, int elo,
-                                                                    int ehi,
-                                                                    int32_t* __restrict__ hist) {
-  __shared__ int cnt[kMaxPermE];
-  const int tid = threadIdx.x;
-  const int64_t lo = (int64_t)blockIdx.x * kPermChunk;
-  const int64_t hi = lo + kPermChunk < P ? lo + kPermChunk : P;
-  for (int e = tid; e < E; e += kPermThreads) cnt[e] = 0;
-  __syncthreads();
-  for (int64_t i = lo + tid; i < hi; i += kPermThreads) {
-    const int e = ids[i];
-    if (e >= elo && e < ehi) atomicAdd(&cnt[e], 1);
-  }
-  __syncthreads();
-  for (int e = tid; e < E; e += kPermThreads) hist[(int64_t)blockIdx.x * E + e] = cnt[e];
-}
-
-__global__ __launch_bounds__(kPermThreads) void permute_scan_kernel(const int32_t* __restrict__ hist,
-                                                                    int nchunks, int E,
-                                                                    int32_t* __restrict__ counts,
-                                                                    int32_t* __restrict__ offsets,
-                                                                    int32_t* __restrict__ starts,
-                                                                    int32_t* __restrict__ zero,
-                                                                    int nzero) {
-  __shared__ int wsum[kPermWaves];
-  const int tid = threadIdx.x;
-  if (zero && tid < nzero) zero[tid] = 0;
-  int v = 0;
-  if (tid < E)
-    for (int c = 0; c < nchunks; ++c) v += hist[(int64_t)c * E + tid];
-  const int excl = block_exclusive_scan(v, wsum);
-  if (tid < E) {
-    counts[tid] = v;
-    offsets[tid] = excl;
-    int run = excl;
-    for (int c = 0; c < nchunks; ++c) {
-      const int h = hist[(int64_t)c * E + tid];
-      starts[(int64_t)c * E + tid] = run;
-      run += h;
-    }
-  }
-  if (tid == E - 1) offsets[E] = excl + v;
-}
+// Larger inputs: chunks of slots, one workgroup each, in two launches: (1) each
+// chunk ranks its slots among the chunk's slots of the same expert (-> slot_pos)
+// and leaves its histogram in table[c * E + e]; (2) each chunk's workgroup sums
+// the histograms of all chunks (-> counts / offsets) and of those before it,
+// which gives its start per expert, and places its slots.  The single workgroup
+// above walks its rounds of 1024 slots one after the other, 2.2 us each.  The
+// table is the caller's scratch, P ints; without one it lies in sorted_slot,
+// which a third launch then fills from slot_pos (the caller makes the chunks so
+// large that chunks * E <= P).  Chunks are a whole number of rounds, at most kPermChunks of
+// them, as every workgroup of (2) reads the whole table.
+constexpr int kPermChunks = 128;
 
 __global__ __launch_bounds__(kPermThreads) void permute_rank_kernel(const int32_t* __restrict__ ids,
-                                                                    int64_t P, int E, int elo,
-                                                                    int ehi,
-                                                                    const int32_t* __restrict__ starts,
+                                                                    int64_t P, int64_t chunk, int E,
+                                                                    int elo, int ehi,
+                                                                    int32_t* __restrict__ table,
                                                                     int32_t* __restrict__ slot_pos) {
   __shared__ int run[kMaxPermE];
   __shared__ int wcnt[kPermWaves][kMaxPermE];
   const int tid = threadIdx.x;
-  const int64_t lo = (int64_t)blockIdx.x * kPermChunk;
-  const int64_t hi = lo + kPermChunk < P ? lo + kPermChunk : P;
+  const int64_t lo = (int64_t)blockIdx.x * chunk;
+  const int64_t hi = lo + chunk < P ? lo + chunk : P;
   for (int e = tid; e < E; e += kPermThreads) {
-    run[e] = starts[(int64_t)blockIdx.x * E + e];
+    run[e] = 0;
     for (int w = 0; w < kPermWaves; ++w) wcnt[w][e] = 0;
   }
   __syncthreads();
   rank_slots(ids, lo, hi, E, elo, ehi, run, wcnt, nullptr, slot_pos);
+  for (int e = tid; e < E; e += kPermThreads) table[(int64_t)blockIdx.x * E + e] = run[e];
+}
+
+// sorted_slot null: slot_pos only
+__global__ __launch_bounds__(kPermThreads) void permute_place_kernel(
+    const int32_t* __restrict__ ids, int64_t P, int64_t chunk, int nchunks, int E, int elo, int ehi,
+    const int32_t* __restrict__ table, int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
+    int32_t* __restrict__ sorted_slot, int32_t* __restrict__ slot_pos, int32_t* __restrict__ zero,
+    int nzero) {
+  __shared__ int all[kPermThreads], before[kPermThreads];
+  __shared__ int start[kMaxPermE];
+  __shared__ int wsum[kPermWaves];
+  const int tid = threadIdx.x, c0 = blockIdx.x;
+  const int64_t lo = (int64_t)c0 * chunk;
+  const int64_t hi = lo + chunk < P ? lo + chunk : P;
+  if (c0 == 0 && zero && tid < nzero) zero[tid] = 0;
+  // the first round's slots are read while the table is summed
+  const int64_t i0 = lo + tid;
+  int e = i0 < hi ? ids[i0] : -1, pos = i0 < hi ? slot_pos[i0] : 0;
+  const int parts = kPermThreads / E;  // threads per expert, each with every parts-th chunk
+  const int part = tid / E, x = tid - part * E;
+  int sum = 0, pre = 0;
+  if (part < parts) {
+#pragma unroll 8
+    for (int c = part; c < nchunks; c += parts) {
+      const int h = table[(int64_t)c * E + x];
+      sum += h;
+      pre += c < c0 ? h : 0;
+    }
+  }
+  all[tid] = sum;
+  before[tid] = pre;
+  __syncthreads();
+  if (tid < E)
+    for (int q = 1; q < parts; ++q) {
+      sum += all[q * E + tid];
+      pre += before[q * E + tid];
+    }
+  else
+    sum = 0;
+  const int excl = block_exclusive_scan(sum, wsum);
+  if (tid < E) {
+    start[tid] = excl + pre;
+    if (c0 == 0) {
+      counts[tid] = sum;
+      offsets[tid] = excl;
+      if (tid == E - 1) offsets[E] = excl + sum;
+    }
+  }
+  __syncthreads();
+  for (int64_t i = i0; i < hi; i += kPermThreads) {
+    if (i != i0) {
+      e = ids[i];
+      pos = slot_pos[i];
+    }
+    if (e >= elo && e < ehi) {
+      pos += start[e];
+      slot_pos[i] = pos;
+      if (sorted_slot) sorted_slot[pos] = (int32_t)i;
+    }
+  }
 }
 
 __global__ __launch_bounds__(256) void permute_scatter_kernel(const int32_t* __restrict__ slot_pos,
@@ -1007,10 +1026,17 @@ int check_moe_shapes(const char* what, int64_t T, int64_t H, int64_t I, int E, i
 
 // Also zeroes zero[0, nzero) (nzero <= 1024) on the way, for the caller's
 // tile counters.  Only the slots whose expert lies in [elo, ehi) are placed
-// (0 <= elo <= ehi <= E; the whole range for a layer on one rank).
+// (0 <= elo <= ehi <= E; the whole range for a layer on one rank).  table: P
+// ints of scratch that no output overlaps, or null.
+//
+// One workgroup or chunks (E = 256, k = 8, one workgroup / chunks with a table /
+// without): 2048 slots 6.5 / 7.1 / 8.7 us, 2400 8.0 / 7.3 / 8.7, 3072 8.5 / 7.4
+// / 8.7, 4096 10.4 / 7.5 / 9.0, 15200 31.7 / 8.5 / 9.9, 65536 126 / 8.9 / 10.4
+// (four launches over chunks of 4096 slots 20.3; 262144 37.1 / here 13.1).
+constexpr int kPermRounds = 2, kPermRoundsNoTable = 3;
 int launch_permute(const int32_t* ids, int64_t T, int k, int E, int32_t* counts, int32_t* offsets,
                    int32_t* sorted_slot, int32_t* slot_pos, int32_t* zero, int nzero,
-                   hipStream_t st, int elo = 0, int ehi = -1) {
+                   int32_t* table, hipStream_t st, int elo = 0, int ehi = -1) {
   if (ehi < 0) ehi = E;
   SGL_REQUIRE(T >= 0 && k >= 1, "moe_permute: bad T=%lld k=%d", (long long)T, k);
   SGL_REQUIRE(E >= 1 && E <= kMaxPermE, "moe_permute: E=%d not in [1, %d]", E,
@@ -1021,20 +1047,26 @@ int launch_permute(const int32_t* ids, int64_t T, int k, int E, int32_t* counts,
   SGL_REQUIRE(counts && offsets && (T == 0 || (ids && sorted_slot && slot_pos)),
               "moe_permute: null pointer");
   const int64_t P = T * k;
-  const int64_t chunks = ceil_div(P, (int64_t)kPermChunk);
-  if (P < 4 * kPermChunk || chunks * E > P) {
+  const int64_t rounds = ceil_div(P, (int64_t)kPermThreads);
+  if (rounds <= (table ? kPermRounds : kPermRoundsNoTable)) {
     permute_kernel<<<1, kPermThreads, 0, st>>>(ids, P, E, counts, offsets, sorted_slot, slot_pos,
                                                zero, nzero, elo, ehi);
     return check_launch("moe_permute");
   }
-  permute_hist_kernel<<<(unsigned)chunks, kPermThreads, 0, st>>>(ids, P, E, elo, ehi, slot_pos);
-  permute_scan_kernel<<<1, kPermThreads, 0, st>>>(slot_pos, (int)chunks, E, counts, offsets,
-                                                       sorted_slot, zero, nzero);
-  permute_rank_kernel<<<(unsigned)chunks, kPermThreads, 0, st>>>(ids, P, E, elo, ehi, sorted_slot,
+  int64_t chunk = ceil_div(rounds, (int64_t)kPermChunks) * kPermThreads;
+  if (ceil_div(P, chunk) * E > P) chunk *= 2;  // chunks * E <= P / 2 + 1024 then, and P > 2048
+  const int64_t chunks = ceil_div(P, chunk);
+  int32_t* tab = table ? table : sorted_slot;
+  permute_rank_kernel<<<(unsigned)chunks, kPermThreads, 0, st>>>(ids, P, chunk, E, elo, ehi, tab,
                                                                   slot_pos);
-  int64_t sblocks = ceil_div(P, (int64_t)256);
-  if (sblocks > 4096) sblocks = 4096;
-  permute_scatter_kernel<<<(unsigned)sblocks, 256, 0, st>>>(slot_pos, P, sorted_slot);
+  permute_place_kernel<<<(unsigned)chunks, kPermThreads, 0, st>>>(
+      ids, P, chunk, (int)chunks, E, elo, ehi, tab, counts, offsets, table ? sorted_slot : nullptr,
+      slot_pos, zero, nzero);
+  if (!table) {
+    int64_t sblocks = ceil_div(P, (int64_t)256);
+    if (sblocks > 4096) sblocks = 4096;
+    permute_scatter_kernel<<<(unsigned)sblocks, 256, 0, st>>>(slot_pos, P, sorted_slot);
+  }
   return check_launch("moe_permute");
 }
 
@@ -1261,7 +1293,7 @@ int sgl_moe_gate(const void* x, const void* w, int64_t T, int64_t H, int E, int 
 int sgl_moe_permute(const int32_t* ids, int64_t T, int k, int E, int32_t* counts, int32_t* offsets,
                     int32_t* sorted_slot, int32_t* slot_pos, sgl_stream_t stream) {
   return sgl::launch_permute(ids, T, k, E, counts, offsets, sorted_slot, slot_pos, nullptr, 0,
-                             (hipStream_t)stream);
+                             nullptr, (hipStream_t)stream);
 }
 
 int sgl_moe_gate_up(const void* xq, const float* xs, int64_t T, int64_t H, int64_t I, int E, int k,
@@ -1359,9 +1391,10 @@ int sgl_moe_forward(const void* x, int64_t T, int64_t H, int64_t I, int E, int k
     a.y = (uint16_t*)y;
     return sgl::launch_small_moe(a, fp4, st);
   }
-  // the permute also zeroes the GEMMs' tile counters
+  // the permute also zeroes the GEMMs' tile counters; its table lies where the
+  // gate/up GEMM writes later (rows * I >= 128 P bytes)
   if ((rc = sgl::launch_permute(ids, T, k, E, w.counts, w.offsets, w.sorted_slot, w.slot_pos,
-                                w.tile_ctr, sgl::kTileCtrs, st)))
+                                w.tile_ctr, sgl::kTileCtrs, (int32_t*)w.hq, st)))
     return rc;
   if ((rc = sgl::run_gate_up(w.xq, w.xs, T, H, I, E, k, w.offsets, w.sorted_slot, weights, experts,
                              has_shared, expert_format, swiglu_limit, scale_mode, w.hq, w.hs,
@@ -1401,7 +1434,8 @@ int sgl_moe_forward_local(const void* x, int64_t T, int64_t H, int64_t I, int E,
   // only the local experts' slots are placed; offsets[E] counts them, and the
   // shared expert's rows follow them as in the whole layer
   if ((rc = sgl::launch_permute(ids, T, k, E, w.counts, w.offsets, w.sorted_slot, w.slot_pos,
-                                w.tile_ctr, sgl::kTileCtrs, st, expert_begin, expert_end)))
+                                w.tile_ctr, sgl::kTileCtrs, (int32_t*)w.hq, st, expert_begin,
+                                expert_end)))
     return rc;
   if ((rc = sgl::run_gate_up(w.xq, w.xs, T, H, I, E, k, w.offsets, w.sorted_slot, weights, experts,
                              has_shared, expert_format, swiglu_limit, scale_mode, w.hq, w.hs,

@@ -226,3 +226,43 @@ def test_router_k_groups(gpu, T, H, E):
     exact = x.astype(np.float64) @ W.astype(np.float64).T
     mag = np.abs(x).astype(np.float64) @ np.abs(W).astype(np.float64).T
     assert np.all(np.abs(f32(lg).astype(np.float64) - exact) <= 2.0 ** -21 * mag + 1e-30)
+
+
+@pytest.mark.parametrize("T,k,E", [
+    (384, 8, 256),    # 3072 slots: the largest of one workgroup
+    (439, 7, 256),    # 3073: four chunks, one slot in the last
+    (700, 6, 1024),   # chunks doubled so that their table fits in the slots, no idle expert thread
+    (5000, 1, 1),     # one expert: every thread sums a part of the table
+    (2001, 3, 1000),  # experts that do not divide the workgroup's threads
+    (16385, 8, 200),  # chunks of two rounds
+])
+def test_permute_chunks(gpu, T, k, E):
+    """The chunked counting sort at its size edges, bit for bit."""
+    from sglang_lite_amd import moe as M
+
+    print(f"permute chunks T={T} k={k} E={E}", flush=True)
+    rng = np.random.default_rng(T + k + E)
+    ids = np.argsort(rng.standard_normal((T, E)) + np.linspace(0, 2, E), axis=1)[:, :k].astype(np.int32)
+    ref = OM.permute(ids, E)
+    for got, name in zip(M.permute(torch.from_numpy(ids).to(gpu), E),
+                         ("counts", "offsets", "sorted_slot", "slot_pos")):
+        np.testing.assert_array_equal(got.cpu().numpy(), ref[name], err_msg=name)
+
+
+@pytest.mark.parametrize("T", [128, 129, 300])
+def test_layer_permute_rounds(gpu, T):
+    """The layer on both sides of the chunked sort's threshold (2048 slots),
+    with the table in its workspace."""
+    from sglang_lite_amd import moe as M
+
+    print(f"layer permute T={T}", flush=True)
+    rng = np.random.default_rng(T)
+    H, I, E, k = 256, 256, 20, 16
+    ids = np.argsort(rng.standard_normal((T, E)), axis=1)[:, :k].astype(np.int32)
+    x = bf16_values(rng, (T, H))
+    w = rng.uniform(0.1, 1.0, (T, k)).astype(np.float32)
+    experts = [OM.make_expert(rng, H, I) for _ in range(E)]
+    sh = OM.make_expert(rng, H, I)
+    y = M.moe_forward(to_dev_bf16(x, gpu), torch.from_numpy(ids).to(gpu), to_dev_f32(w, gpu),
+                      table_from(experts, sh, gpu))
+    assert_gemm_close(f32(y), OM.moe_forward(x, ids, w, experts, sh), f"layer permute T={T}")
