@@ -196,11 +196,12 @@ int sgl_mfma_mix_threads(void);
  * [ceil(N/128), K/128] fp32, or one e8m0 byte per scale when b_scale_e8m0 is
  * set.  K % 128 == 0, N % 16 == 0, M*K and N*K < 2^31.
  * Shapes for which sgl_fp8_gemm_workspace_size is non-zero (16 < M <= 64
- * with N % 128 == 0) split the K range over workgroups and keep the fp32
- * partials in the caller's workspace (16-byte aligned, at least that many
- * bytes; a smaller one is SGL_ERR_WORKSPACE).  Whether a shape splits
- * depends on the shape alone, so eager and graph-captured calls sum in the
- * same order.  Calls that overlap in time need workspaces of their own.
+ * with N % 128 == 0) need a workspace (16-byte aligned, at least that many
+ * bytes; a smaller one is SGL_ERR_WORKSPACE): where the K range is split over
+ * workgroups it holds the fp32 partials; most of these shapes split K inside
+ * a workgroup instead and leave it untouched.  Which it is depends on the
+ * shape and the kinds of scales alone, so eager and graph-captured calls sum
+ * in the same order.  Calls that overlap in time need workspaces of their own.
  * Replaces deepseek_infer/kernel.py:257-273 fp8_gemm (kernel :203-254) and the
  * call-site adapter engine/v4_deep_gemm.py:169-218 fp4_gemm_nt (whose
  * workspace-free call the reference's adapter allocates with torch at
@@ -345,6 +346,8 @@ size_t sgl_moe_workspace_size(int64_t T, int64_t H, int64_t I, int E, int k, int
 /* Whole routed+shared MoE layer from bf16 x [T, H] and a precomputed top-k
  * (ids int32 [T, k], weights fp32 [T, k]): act quant -> permute -> gate/up
  * -> down -> combine, y bf16 [T, H]; routed experts in expert_format.
+ * The smallest batches (FP4 T*k <= 24, FP8 T = 1 or T*k <= 8) run gate/up and
+ * down without a permute or combine; the same rounding points and workspace.
  * Replaces engine/v4_moe_fast.py:79-106 _moe_forward_activated_only after
  * the gate.  Every launch goes to `stream`. */
 int sgl_moe_forward(const void* x, int64_t T, int64_t H, int64_t I, int E, int k,
@@ -438,7 +441,7 @@ enum sgl_attn_kv_format {
 
 /* Sparse multi-head attention with an attention sink over gathered KV rows:
  * for query (b, m) and head h, s_j = (q[b,m,h] . kv[b, idx[b,m,j]]) * scale
- * (idx -1, or outside [0, n), masked), online softmax over blocks of 64 rows
+ * (idx -1, or outside [0, n), masked), online softmax over blocks of rows
  * with bf16 probabilities in the P.V product and fp32 ones in the normaliser,
  * o = acc / (sum + exp(attn_sink[h] - max)) as bf16.  q bf16 [B, M, Hh, 512],
  * o bf16 [B, M, Hh, 512], attn_sink fp32 [Hh], topk_idxs int32 [B, M, K]; the

@@ -2796,8 +2796,8 @@ int launch_cfg(GemmArgs& a, hipStream_t stream) {
 #ifndef SGL_SKINNY_MAX_M
 #define SGL_SKINNY_MAX_M 64
 #endif
-// dense GEMMs up to this M take the skinny kernel (measured crossover with
-// the 64 x 128 tiles)
+// dense GEMMs up to this M take the skinny kernel where neither split-K nor
+// the K-group tiles apply (measured crossover with the 64 x 128 tiles)
 constexpr int64_t kSkinnyMaxM = SGL_SKINNY_MAX_M;
 template <int TM>
 struct Skinny {
@@ -2997,10 +2997,11 @@ int launch_skinny(GemmArgs& a, hipStream_t stream) {
 // promoted with sa sb in fp32, as everywhere).  The fp32 tile partials go to
 // a workspace and splitk_reduce_kernel, over the whole GPU, sums them in split
 // order: C is the same bytes on every run.  (N = 4096, K = 7168 at M = 64: 12
-// us + 4 us, against 22.6 us for the unsplit kernel.  At M <= 32 the unsplit
-// kernel reads less A and already runs near a read-only stream of B, and the
-// reduction does not pay: a last-workgroup sum costs three dependent trips to
-// device-coherent memory, about 3 us.)
+// us + 4 us, against 22.6 us for the skinny kernel.  A last-workgroup sum in
+// place of the second launch costs three dependent trips to device-coherent
+// memory, about 3 us.)  The tiles that split K inside a workgroup need no
+// partials and take the shape wherever they cover the CUs (11.8 us there with
+// e8m0 scales, split-K 14.7); this is what is left: few tiles, or fp32 scales.
 namespace splitk {
 constexpr int NW = 8, NT = 64 * NW, BN = 16 * NW, KSMAX = 8, SMAX = 16, TMMAX = 4;
 }  // namespace splitk
@@ -3232,8 +3233,9 @@ int launch_splitk_tm(GemmArgs& a, int KS, int S, float* part, hipStream_t stream
   }
 }
 
-// The split of a dense FP8 GEMM over K, a function of the shape alone (so an
-// eager call and a captured one sum in the same order): 16 < M <= 64
+// The split of a dense FP8 GEMM over K, and the workspace a call must bring, a
+// function of the shape alone (so an eager call and a captured one sum in the
+// same order): 16 < M <= 64
 // (N = 4096, K = 7168, graph-replayed over cold weights: M = 32 12.1 us where
 // the skinny kernel takes 14.3; M = 16 10.9 vs 10.5, M = 128 with 128-row
 // tiles 23.0 vs 22.0 with 32 x 64 tiles), N % 128 == 0, about one workgroup
