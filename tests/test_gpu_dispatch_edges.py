@@ -177,6 +177,21 @@ def test_sparse_attn_row_list_edges(gpu, fmt, K, queries):
         assert_gemm_close(got[:, s:s + 1], ref, f"K={K} query {s}")
 
 
+@pytest.mark.parametrize("queries", [8, 9, 24])
+@pytest.mark.parametrize("H", [6, 64, 70])
+def test_sparse_attn_merge_order(gpu, queries, H):
+    """Split rows merged on both orders of workgroups (a multiple of eight
+    queries or not), head counts that do not fill a workgroup's four."""
+    rng = np.random.default_rng(queries + H)
+    K = 1024
+    print(f"attn merge H={H} queries={queries}", flush=True)
+    q, kv = bf16_values(rng, (1, queries, H, 512)), bf16_values(rng, (1, 60, 512))
+    sink = rng.standard_normal(H).astype(np.float32)
+    idx = rng.integers(0, 60, (1, queries, K)).astype(np.int32)
+    got, rows = _attn(gpu, q, kv, sink, idx, 512 ** -0.5, "bf16")
+    assert_gemm_close(got, OA.sparse_attn_blocked(q, rows, sink, idx, 512 ** -0.5), f"H={H} queries={queries}")
+
+
 @pytest.mark.parametrize("order", ["rising", "falling", "one late"])
 def test_sparse_attn_moving_reference(gpu, order):
     """Scores that rise block after block (the reference moves in each), fall,
