@@ -55,6 +55,7 @@
 
 #include "sgl_common.h"
 #include "sgl_numeric.h"
+#include "sgl_rules.h"
 
 namespace sgl {
 namespace {
@@ -174,8 +175,7 @@ __device__ __forceinline__ void attn_role(const AttnArgs& a, Smem<FMT>& sm) {
   const int wo = wave & 3;                        // O: dims [128 wo, +128)
   const int l16 = lane & 15, g4 = lane >> 4;
   const int g2 = lane >> 5, c32 = lane & 31;
-  // later queries of a prefill select more rows: they start first
-  const int64_t m = a.M - 1 - (int64_t)blockIdx.x, b = blockIdx.y;
+  const int64_t m = attn_query_in_seq(blockIdx.x, (uint32_t)a.M), b = blockIdx.y;
   const int split = (int)(blockIdx.z % a.nsplit);
   const int h0 = (int)(blockIdx.z / a.nsplit) * kHG;
   const int nh = min(a.Hh - h0, kHG);             // heads of this group
@@ -687,27 +687,13 @@ void sparse_attn_kernel(const AttnArgs a) {
 // log2 units:
 //   M = max_s m_s;  o = sum_s acc_s 2^(m_s - M) / (sum_s l_s 2^(m_s - M) + e^(sink) 2^(-M))
 // (splits whose rows were all masked carry m = -inf and add nothing).
-// Workgroups go round the eight XCDs in order, so with a multiple of eight
-// queries every split of query q ran on XCD q % 8; its merge goes there too and
-// finds the partials in that L2, and the next call's partials overwrite lines
-// that this L2 alone holds (32 sequences x 640 rows: the attention kernel
-// 21.9 -> 19.2 us, the merge 5.4 -> 4.3, a call 27.5 -> 22.4).
-__global__ __launch_bounds__(256) void sparse_attn_combine_kernel(const AttnArgs a, int64_t queries) {
+__global__ __launch_bounds__(256) void sparse_attn_combine_kernel(const AttnArgs a, uint32_t queries) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  int64_t q;  // b * M + m
-  int h;
-  if (queries % 8 == 0) {
-    const int per = (a.Hh + 3) >> 2;  // workgroups of a query, four heads each
-    const int64_t i = blockIdx.x >> 3;
-    q = 8 * (i / per) + (blockIdx.x & 7);
-    h = 4 * (int)(i % per) + wave;
-  } else {
-    const int64_t w = (int64_t)blockIdx.x * 4 + wave;
-    q = w / a.Hh;
-    h = (int)(w % a.Hh);
-  }
-  if (q >= queries || h >= a.Hh) return;
+  const AttnMerge at = attn_merge_at(blockIdx.x, wave, queries, (uint32_t)a.M, (uint32_t)a.Hh);
+  if (at.query >= queries || at.head >= (uint32_t)a.Hh) return;
+  const int64_t q = at.query;  // b * M + m
+  const int h = (int)at.head;
   const int64_t w = q * a.Hh + h;
   const float NEG_INF = -__builtin_huge_valf();
   // every split's loads are issued before the first is used (at most
@@ -858,9 +844,9 @@ extern "C" int sgl_sparse_attn(const void* q, int64_t B, int64_t M, int Hh, cons
     SGL_ATTN(SGL_ATTN_KV_A_PAGED);
 #undef SGL_ATTN
   if (a.nsplit > 1) {
-    const int64_t Q = B * M;
-    const int64_t groups = Q % 8 == 0 ? Q * sgl::ceil_div(Hh, 4) : sgl::ceil_div(Q * Hh, (int64_t)4);
-    sgl::sparse_attn_combine_kernel<<<(unsigned)groups, 256, 0, st>>>(a, Q);
+    // (more than one split: fewer queries x head groups than CUs)
+    const uint32_t Q = (uint32_t)(B * M);
+    sgl::sparse_attn_combine_kernel<<<sgl::attn_merge_groups(Q, (uint32_t)Hh), 256, 0, st>>>(a, Q);
   }
   return sgl::check_launch("sparse_attn");
 }

@@ -1,0 +1,59 @@
+"""The size rules of the dispatches (csrc/sgl_rules.h), compiled for the host."""
+
+from __future__ import annotations
+
+import ctypes
+import subprocess
+from pathlib import Path
+
+import pytest
+
+CSRC = Path(__file__).resolve().parents[1] / "sglang-lite_amd" / "csrc"
+
+WRAPPERS = r"""
+#include "sgl_rules.h"
+using namespace sgl;
+extern "C" {
+// the query of a workgroup of the attention grid (M, B, z), as its kernel names it
+uint32_t attn_query(uint32_t x, uint32_t y, uint32_t M) { return y * M + attn_query_in_seq(x, M); }
+uint32_t merge_groups(uint32_t queries, uint32_t heads) { return attn_merge_groups(queries, heads); }
+void merge_at(uint32_t wg, uint32_t wave, uint32_t queries, uint32_t M, uint32_t heads, uint32_t* out) {
+  const AttnMerge m = attn_merge_at(wg, wave, queries, M, heads);
+  out[0] = m.query;
+  out[1] = m.head;
+}
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    d = tmp_path_factory.mktemp("rules")
+    src, so = d / "rules.cpp", d / "rules.so"
+    src.write_text(WRAPPERS)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-O1", "-shared", "-fPIC", f"-I{CSRC}",
+                    str(src), "-o", str(so)], check=True)
+    return ctypes.CDLL(str(so))
+
+
+@pytest.mark.parametrize("B,M", [(32, 1), (1, 8), (4, 8), (8, 4), (4, 2), (16, 3), (3, 16), (1, 24), (7, 1), (3, 3)])
+@pytest.mark.parametrize("heads", [1, 6, 64, 70])
+def test_attention_merge_covers_and_follows_the_splits(rules, B, M, heads):
+    """Every (query, head) is merged once; with a multiple of eight queries by
+    a workgroup of the XCD (linear workgroup index mod 8) of its splits."""
+    Q = B * M
+    ran_on = {rules.attn_query(x, y, M): (x + M * y) % 8 for y in range(B) for x in range(M)}
+    assert sorted(ran_on) == list(range(Q))  # (split and head group z: x + M (y + B z), the same mod 8 if 8 | Q)
+    seen = set()
+    out = (ctypes.c_uint32 * 2)()
+    for wg in range(rules.merge_groups(Q, heads)):
+        for wave in range(4):
+            rules.merge_at(wg, wave, Q, M, heads, out)
+            q, h = out[0], out[1]
+            if q >= Q or h >= heads:
+                continue
+            assert (q, h) not in seen
+            seen.add((q, h))
+            if Q % 8 == 0:
+                assert ran_on[q] == wg % 8, f"query {q}"
+    assert len(seen) == Q * heads
