@@ -51,8 +51,6 @@
 // (640 indices, -1 where a token has fewer rows) 320 -> 182 us.  The roles
 // without the MFMAs between reads and gathers (each fragment read waited for
 // by itself): 1.3 us a block.
-#include <algorithm>
-
 #include "sgl_common.h"
 #include "sgl_numeric.h"
 #include "sgl_rules.h"
@@ -67,9 +65,8 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 typedef v4s __attribute__((address_space(3))) lds_v4s;
 
 constexpr int kD = 512;     // head dim: 448 latent + 64 rope
-constexpr int kBlk = 64;    // gathered rows per block
+constexpr int kBlk = 64;    // indices a split is cut by
 constexpr int kHG = 64;     // heads per workgroup
-constexpr int kMaxSplits = 8;  // workgroups a query's rows split over, at most
 constexpr int kARow = 584, kAData = 576, kANope = 448;
 constexpr float kLog2e = 1.4426950408889634f;
 
@@ -697,12 +694,12 @@ __global__ __launch_bounds__(256) void sparse_attn_combine_kernel(const AttnArgs
   const int64_t w = q * a.Hh + h;
   const float NEG_INF = -__builtin_huge_valf();
   // every split's loads are issued before the first is used (at most
-  // kMaxSplits splits), so their latencies overlap instead of adding up;
+  // kAttnMaxSplits splits), so their latencies overlap instead of adding up;
   // the maximum and the sums then run in split order as before
-  float msp[kMaxSplits], lsp[kMaxSplits];
-  float4 usp[kMaxSplits], vsp[kMaxSplits];
+  float msp[kAttnMaxSplits], lsp[kAttnMaxSplits];
+  float4 usp[kAttnMaxSplits], vsp[kAttnMaxSplits];
 #pragma unroll
-  for (int sp = 0; sp < kMaxSplits; ++sp) {
+  for (int sp = 0; sp < kAttnMaxSplits; ++sp) {
     if (sp < a.nsplit) {
       const int64_t r = (q * a.nsplit + sp) * a.Hh + h;
       msp[sp] = a.ws_ml[r * 2];
@@ -714,13 +711,13 @@ __global__ __launch_bounds__(256) void sparse_attn_combine_kernel(const AttnArgs
   }
   float mx = NEG_INF;
 #pragma unroll
-  for (int sp = 0; sp < kMaxSplits; ++sp)
+  for (int sp = 0; sp < kAttnMaxSplits; ++sp)
     if (sp < a.nsplit) mx = fmaxf_(mx, msp[sp]);
   const float ref = mx == NEG_INF ? 0.0f : mx;
   float o[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   float l = 0.0f;
 #pragma unroll
-  for (int sp = 0; sp < kMaxSplits; ++sp) {
+  for (int sp = 0; sp < kAttnMaxSplits; ++sp) {
     if (sp < a.nsplit) {
       const float f = __builtin_amdgcn_exp2f(msp[sp] - ref);  // 0 for an all-masked split
       l += lsp[sp] * f;
@@ -736,41 +733,12 @@ __global__ __launch_bounds__(256) void sparse_attn_combine_kernel(const AttnArgs
   *reinterpret_cast<uint4*>(a.o + w * (int64_t)kD + lane * 8) = make_uint4(wv[0], wv[1], wv[2], wv[3]);
 }
 
-// Splits of the gathered rows: at most enough workgroups to give every CU one,
-// at most one split per 64-row block and kMaxSplits.  A split shortens the
-// serial chain of blocks but writes an fp32 partial of all its heads (128 KB
-// per 64 heads) that the merge reads back, so it is taken where the chain it
-// saves costs more than that.  In tenths of a us, fitted to 1 / 8 / 32 / 64
-// sequences x 128 ... 2048 rows with 1 to 8 splits: a 64-row block 18 (bf16)
-// or 24 (FP8), a merge 26 plus 0.8 per partial, at most 116.  (64 sequences x 128
-// rows: one split 11.7 us, two 22.7; 32 x 640: five 23.8, two 24.7, one 26.6.)
-int attn_splits(int64_t B, int64_t M, int Hh, int64_t K, bool fp8) {
-  const int64_t wgs = B * M * ((Hh + kHG - 1) / kHG);
-  const int64_t nblk = (K + kBlk - 1) / kBlk;
-  int64_t most = (device_cu_count() + wgs - 1) / (wgs > 0 ? wgs : 1);
-  if (most > nblk) most = nblk;
-  if (most > kMaxSplits) most = kMaxSplits;
-  int best = 1;
-  int64_t best_cost = nblk * (fp8 ? 240 : 180);
-  for (int64_t want = 2; want <= most; ++want) {
-    const int64_t bps = (nblk + want - 1) / want, ns = (nblk + bps - 1) / bps;  // no empty split
-    const int64_t parts = 8 * wgs * ns;
-    const int64_t cost = bps * (fp8 ? 240 : 180) + 260 + (parts < 900 ? parts : 900);
-    if (cost < best_cost) {
-      best_cost = cost;
-      best = (int)ns;
-    }
-  }
-  return best;
-}
-
 }  // namespace
 }  // namespace sgl
 
 extern "C" size_t sgl_sparse_attn_workspace_size(int64_t B, int64_t M, int Hh, int64_t K) {
   if (B <= 0 || M <= 0 || Hh <= 0 || K <= 0) return 0;
-  // enough for any kv_format
-  const int ns = std::max(sgl::attn_splits(B, M, Hh, K, false), sgl::attn_splits(B, M, Hh, K, true));
+  const int ns = sgl::attn_splits(B * M, Hh, K, sgl::device_cu_count());
   if (ns == 1) return 0;
   return (size_t)(B * M * ns * Hh) * (sgl::kD + 2) * 4;
 }
@@ -811,7 +779,7 @@ extern "C" int sgl_sparse_attn(const void* q, int64_t B, int64_t M, int Hh, cons
   a.Hh = Hh;
   a.scale = softmax_scale;
   a.o = (uint16_t*)o;
-  a.nsplit = K > 0 ? sgl::attn_splits(B, M, Hh, K, kv_format != SGL_ATTN_KV_BF16) : 1;
+  a.nsplit = sgl::attn_splits(B * M, Hh, K, sgl::device_cu_count());
   const int64_t nblk = (K + sgl::kBlk - 1) / sgl::kBlk;
   a.bps = (int)((nblk + a.nsplit - 1) / a.nsplit);
   a.ws_acc = nullptr;

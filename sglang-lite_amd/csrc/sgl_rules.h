@@ -46,4 +46,40 @@ SGL_RULE AttnMerge attn_merge_at(uint32_t wg, uint32_t wave, uint32_t queries, u
   return {w / heads, w % heads};
 }
 
+// ---- sparse attention: the workgroups (splits) that share a query's K
+// indices, cut in 64s: at most one a CU, at most kAttnMaxSplits.  A function of
+// the shape alone and not of the cache's format, so that the packed cache gives
+// bit for bit what its dequantized rows give.
+//
+// A split shortens the serial chain of blocks but writes fp32 partials (128 KB
+// per 64 heads) that a merge reads back.  The cheapest by these costs, in
+// 1/100 us, fitted to 1 ... 256 queries x 64 ... 2048 indices x 1 ... 128 heads,
+// bf16 rows and packed pages, every number of splits:
+//   a block of 64 indices: 250;
+//   a merge: 140 and 31 a split, up to 88 more with the heads, and for each
+//     partial of 64 heads 4.5 where the merge follows its splits (a multiple of
+//     eight queries), else 7.2, at most 990.
+// (64 heads, packed pages, us: 32 / 33 queries x 128 indices, one split / two
+// 15.2 / 17.4 and 15.1 / 20.7; 32 x 384, one / three 25.3 / 20.8; 32 x 640, one
+// / five 35.6 / 23.5; 33 x 2048, seven 36.7, eight, which are 264 workgroups,
+// 52.6.)
+constexpr int kAttnMaxSplits = 8;
+SGL_RULE int attn_splits(int64_t queries, int heads, int64_t K, int cus) {
+  const int64_t blocks = (K + 63) / 64, wgs = queries * ((heads + 63) / 64);
+  const int64_t h64 = heads < 64 ? heads : 64;
+  int best = 1;
+  int64_t best_cost = blocks * 250;
+  for (int64_t want = 2; want <= kAttnMaxSplits && want <= blocks && want * wgs <= cus; ++want) {
+    const int64_t bps = (blocks + want - 1) / want, ns = (blocks + bps - 1) / bps;  // no empty split
+    int64_t parts = queries * ns * heads * (queries % 8 == 0 ? 45 : 72) / 640;
+    if (queries % 8 != 0 && parts > 990) parts = 990;
+    const int64_t cost = bps * 250 + 140 + 31 * ns + 88 * h64 / 64 + parts;
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = (int)ns;
+    }
+  }
+  return best;
+}
+
 }  // namespace sgl

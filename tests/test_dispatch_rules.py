@@ -22,6 +22,7 @@ void merge_at(uint32_t wg, uint32_t wave, uint32_t queries, uint32_t M, uint32_t
   out[0] = m.query;
   out[1] = m.head;
 }
+int splits(int64_t queries, int heads, int64_t K, int cus) { return attn_splits(queries, heads, K, cus); }
 }
 """
 
@@ -57,3 +58,20 @@ def test_attention_merge_covers_and_follows_the_splits(rules, B, M, heads):
             if Q % 8 == 0:
                 assert ran_on[q] == wg % 8, f"query {q}"
     assert len(seen) == Q * heads
+
+
+@pytest.mark.parametrize("cus", [256, 64, 1])
+def test_attention_splits_fit_the_device(rules, cus):
+    """At most a workgroup per CU once a query is split, none of them empty."""
+    i64 = ctypes.c_int64
+    for queries in (1, 7, 8, 32, 33, 100, 128, 129, 256, 5000):
+        for heads in (1, 8, 64, 65, 128):
+            for K in (0, 1, 64, 65, 192, 640, 2048, 100000):
+                ns = rules.splits(i64(queries), heads, i64(K), cus)
+                blocks = -(-K // 64)
+                assert 1 <= ns <= 8
+                if ns > 1:
+                    assert ns * queries * -(-heads // 64) <= cus
+                    assert ns <= blocks and (ns - 1) * -(-blocks // ns) < blocks
+    assert rules.splits(i64(32), 64, i64(640), 256) == 5
+    assert rules.splits(i64(33), 64, i64(2048), 256) == 7

@@ -281,3 +281,21 @@ def test_layer_permute_rounds(gpu, T):
     y = M.moe_forward(to_dev_bf16(x, gpu), torch.from_numpy(ids).to(gpu), to_dev_f32(w, gpu),
                       table_from(experts, sh, gpu))
     assert_gemm_close(f32(y), OM.moe_forward(x, ids, w, experts, sh), f"layer permute T={T}")
+
+
+@pytest.mark.parametrize("queries,H,K", [(8, 64, 192), (16, 64, 256), (32, 64, 384), (33, 64, 384), (32, 8, 256),
+                                         (64, 16, 384), (33, 100, 640), (300, 64, 200)])
+def test_sparse_attn_formats_split_alike(gpu, queries, H, K):
+    """Packed rows and pages give bit for bit what their dequantized rows give,
+    at sizes where one split or several are close."""
+    rng = np.random.default_rng(queries + H + K)
+    print(f"attn formats queries={queries} H={H} K={K}", flush=True)
+    n = 96
+    q, kv = bf16_values(rng, (1, queries, H, 512)), bf16_values(rng, (1, n, 512))
+    sink = rng.standard_normal(H).astype(np.float32)
+    idx = rng.integers(-1, n, (1, queries, K)).astype(np.int32)
+    got, rows = _attn(gpu, q, kv, sink, idx, 512 ** -0.5, "rows")
+    paged, _ = _attn(gpu, q, kv, sink, idx, 512 ** -0.5, "pages")
+    plain, _ = _attn(gpu, q, rows, sink, idx, 512 ** -0.5, "bf16")
+    np.testing.assert_array_equal(got, plain)
+    np.testing.assert_array_equal(paged, plain)
