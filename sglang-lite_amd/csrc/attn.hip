@@ -133,8 +133,10 @@ constexpr int kTile = kRows * 1024;  // bytes of a row-major bf16 tile
 constexpr int kRing = 4;             // tiles
 constexpr int kPTile = kHG * 64;     // bytes of P: [head][32 tokens] bf16
 
-// Selected rows held in LDS at a time (a multiple of 64): their addresses
-// and, FP8, the distance to their scale bytes.
+// Selected rows held in LDS at a time: their addresses and, FP8, the distance
+// to their scale bytes.  A list that is not the last runs its whole blocks and
+// leaves the rest to the next, so that the blocks (and with them the rounding)
+// do not depend on its length.
 template <int FMT>
 constexpr int kList = FMT == SGL_ATTN_KV_BF16 ? 2752 : 1792;
 
@@ -147,6 +149,7 @@ struct Smem {
   float mx[2][kHG];                       // block maxima per token half and head (then the sums)
   float sink[kHG];                        // log2 units
   int flag[4];                            // block n's at n % 4: a score above its reference
+  int64_t next;                           // index the next list starts at, -1: this is the last
 };
 
 __device__ const uint4 g_zero_row[64] = {};  // what a block's rows past the list read
@@ -230,14 +233,13 @@ __device__ __forceinline__ void attn_role(const AttnArgs& a, Smem<FMT>& sm) {
 
   int moves = 0;  // of the references
   bool first = true;
-  for (int64_t kc = k_begin; kc < k_end || first; kc += kList<FMT>) {
-    // ---- the chunk's valid rows, packed in order, padded to a whole block.
-    // Every wavefront writes the whole list (the same values), so each reads
-    // back its own writes
-    if (!first) __syncthreads();  // the previous chunk's list and tiles are consumed
+  for (int64_t kc = k_begin;;) {
+    // ---- the valid rows from index kc on, packed in order, the last list
+    // padded to a whole block.  Every wavefront writes the whole list (the same
+    // values), so each reads back its own writes
+    if (!first) __syncthreads();  // the previous list and tiles are consumed
     if (threadIdx.x < 4) sm.flag[threadIdx.x] = 0;
     int cnt = 0;
-    const int64_t ke = min(kc + (int64_t)kList<FMT>, k_end);
     auto put_row = [&](int at, int id) {
       if constexpr (kDma) {
         sm.row[at] = (uint64_t)(uintptr_t)kvb + (uint64_t)(uint32_t)id * ((uint64_t)a.ld * 2);
@@ -251,29 +253,49 @@ __device__ __forceinline__ void attn_role(const AttnArgs& a, Smem<FMT>& sm) {
         sm.foot[at] = kAData;
       }
     };
-    for (int64_t p0 = kc; p0 < ke; p0 += 4 * 64) {
+    auto before = [](uint64_t mask) -> int {  // set bits below this lane
+      return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
+    };
+    int64_t pe = kc;  // end of the indices taken
+    int li = lane;  // made opaque, so that no address made from it is kept in registers across the phases
+    asm volatile("" : "+v"(li));
+    while (pe < k_end && cnt + 64 <= kList<FMT>) {
       int32_t id[4];
+      const int64_t p0 = pe;
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const int64_t p = p0 + u * 64 + lane;
-        id[u] = idxp[p < ke ? p : ke - 1];
+        const int64_t p = p0 + u * 64 + li;
+        id[u] = idxp[p < k_end ? p : k_end - 1];
       }
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const bool ok = p0 + u * 64 + lane < ke && id[u] >= 0 && id[u] < a.n;
+        if (cnt + 64 > kList<FMT>) break;
+        const bool ok = p0 + u * 64 + li < k_end && id[u] >= 0 && id[u] < a.n;
         const uint64_t mask = __ballot(ok);
-        const int before = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
-                                                     __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
-        if (ok) put_row(cnt + before, id[u]);
-        cnt += __popcll(mask);
+        if (ok) put_row(cnt + before(mask), id[u]);
+        cnt = __builtin_amdgcn_readfirstlane(cnt + __popcll(mask));
+        pe = p0 + (u + 1) * 64;
       }
     }
-    cnt = __builtin_amdgcn_readfirstlane(cnt);
-    if (lane < kRows) {  // (read only when cnt > 0: row 0 exists)
-      if constexpr (kDma) sm.row[cnt + lane] = (uint64_t)(uintptr_t)g_zero_row;
-      else put_row(cnt + lane, 0);
+    if (li < kRows) {  // (read only when cnt > 0: row 0 exists)
+      if constexpr (kDma) sm.row[cnt + li] = (uint64_t)(uintptr_t)g_zero_row;
+      else put_row(cnt + li, 0);
     }
-    const int nblk = (cnt + kRows - 1) / kRows;
+    const bool last = pe >= k_end;
+    const int nblk = (last ? cnt + kRows - 1 : cnt) / kRows;
+    if (!last) {  // the next list starts at the first row left over
+      int left = cnt - nblk * kRows;  // (a list that is not the last has more than a block)
+      while (left > 0) {
+        pe -= 64;
+        const int32_t id = idxp[pe + li];
+        const bool ok = id >= 0 && id < a.n;
+        const uint64_t mask = __ballot(ok);
+        const int here = __popcll(mask);
+        if (here >= left) pe += __builtin_ctzll(__ballot(ok && before(mask) == here - left));
+        left = here >= left ? 0 : left - here;
+      }
+    }
+    sm.next = last ? -1 : pe;  // (kept here, not in the scalar registers, which the phases need)
 
     // ---- row gathers: rows 8 wo + rr of a block, by the O wavefronts (the
     // first time the S wavefronts take block 1).  bf16: one DMA per row, lane
@@ -593,7 +615,10 @@ __device__ __forceinline__ void attn_role(const AttnArgs& a, Smem<FMT>& sm) {
         }
       }
     }
-    if (kc >= k_end) break;  // no indices at all
+    const int2 next = *reinterpret_cast<const int2*>(&sm.next);
+    const int next_hi = __builtin_amdgcn_readfirstlane(next.y);
+    if (next_hi < 0) break;
+    kc = (int64_t)next_hi << 32 | (uint32_t)__builtin_amdgcn_readfirstlane(next.x);
   }
 
   // ---- the heads' sums meet in LDS; the outputs pass through the tiles so

@@ -284,7 +284,8 @@ def test_layer_permute_rounds(gpu, T):
 
 
 @pytest.mark.parametrize("queries,H,K", [(8, 64, 192), (16, 64, 256), (32, 64, 384), (33, 64, 384), (32, 8, 256),
-                                         (64, 16, 384), (33, 100, 640), (300, 64, 200)])
+                                         (64, 16, 384), (33, 100, 640), (300, 64, 200),
+                                         (300, 2, 2000), (257, 33, 3600), (1, 64, 20000)])  # lists of several parts
 def test_sparse_attn_formats_split_alike(gpu, queries, H, K):
     """Packed rows and pages give bit for bit what their dequantized rows give,
     at sizes where one split or several are close."""
@@ -299,3 +300,24 @@ def test_sparse_attn_formats_split_alike(gpu, queries, H, K):
     plain, _ = _attn(gpu, q, rows, sink, idx, 512 ** -0.5, "bf16")
     np.testing.assert_array_equal(got, plain)
     np.testing.assert_array_equal(paged, plain)
+
+
+@pytest.mark.parametrize("valid", [1727, 1728, 1729, 1792, 1793, 2688, 2752, 2753, 3600])
+@pytest.mark.parametrize("K", [3600, 5000])
+def test_sparse_attn_row_lists_by_valid_rows(gpu, valid, K):
+    """Valid rows that fill the list (1792 packed, 2752 bf16) or pass it, between
+    masked entries: the formats bit for bit, and the exact softmax."""
+    rng = np.random.default_rng(valid + K)
+    print(f"attn lists valid={valid} K={K}", flush=True)
+    S, H, n = 257, 2, 64
+    q, kv = bf16_values(rng, (1, S, H, 512)), bf16_values(rng, (1, n, 512))
+    sink = rng.standard_normal(H).astype(np.float32)
+    idx = np.full((1, S, K), -1, np.int32)
+    for s in range(S):
+        idx[0, s, np.sort(rng.permutation(K)[:valid])] = rng.integers(0, n, valid)
+    got, rows = _attn(gpu, q, kv, sink, idx, 512 ** -0.5, "rows")
+    plain, _ = _attn(gpu, q, rows, sink, idx, 512 ** -0.5, "bf16")
+    np.testing.assert_array_equal(got, plain)
+    for s in (0, S - 1):
+        ref = OA.sparse_attn_exact(q[:, s:s + 1], rows, sink, idx[:, s:s + 1], 512 ** -0.5)
+        assert_gemm_close(got[:, s:s + 1], ref, f"valid={valid} query {s}")
