@@ -106,9 +106,15 @@ __device__ __forceinline__ uint32_t cvt2_e4m3_bf16(uint32_t w, float sc) {
 }
 
 // 16 bytes at an 8-byte aligned address (layout A rows)
-struct __attribute__((packed, aligned(8))) U4a8 {
-  uint32_t x, y, z, w;
-};
+typedef uint32_t V4a8 __attribute__((ext_vector_type(4), aligned(8)));
+
+// A load from device memory at a 64-bit address: as a global load, since a flat
+// one would count as LDS traffic too and be waited for at every barrier.
+template <typename T>
+__device__ __forceinline__ T ld_global(uint64_t addr) {
+  typedef const T __attribute__((address_space(1))) gT;
+  return *(gT*)(uintptr_t)addr;
+}
 
 // Barrier behind this wavefront's own LDS traffic and, with VM, its DMAs
 // (which the compiler does not count).  The register loads the compiler
@@ -312,14 +318,14 @@ __device__ __forceinline__ void attn_role(const AttnArgs& a, Smem<FMT>& sm) {
                 kv_lds + (uint32_t)((j & (kRing - 1)) * kTile + wo * 8192 + rr * 1024), j, nblk);
     };
     struct Raw {  // FP8 rows on their way: two per pair
-      U4a8 nope[kDma ? 1 : 4], rope;
+      V4a8 nope[kDma ? 1 : 4], rope;
       uint32_t sc[kDma ? 1 : 4];
     } raw;
     auto load_pair = [&](int at, int p, Raw& w) {
       const int lc = min(ln, 55), half = lc >= 28, piece = lc - 28 * half;
       const uint64_t row = sm.row[at + 2 * p + half];
-      w.nope[p] = *reinterpret_cast<const U4a8*>((uintptr_t)(row + 16 * piece));
-      w.sc[p] = *reinterpret_cast<const uint8_t*>((uintptr_t)(row + sm.foot[at + 2 * p + half] + (piece >> 2)));
+      w.nope[p] = ld_global<V4a8>(row + 16 * piece);
+      w.sc[p] = ld_global<uint8_t>(row + sm.foot[at + 2 * p + half] + (piece >> 2));
     };
     auto store_pair = [&](int j, int p, const Raw& w) {
       const int lc = min(ln, 55), half = lc >= 28, piece = lc - 28 * half;
@@ -327,7 +333,7 @@ __device__ __forceinline__ void attn_role(const AttnArgs& a, Smem<FMT>& sm) {
       const uint32_t off = (uint32_t)((j & (kRing - 1)) * kTile + wo * 8192 + p * 2048) +
                            ((uint32_t)(half * 1024 + ((2 * piece) ^ (half << 2)) * 16) ^ (c << 4));
       const float sc = bits_f32(w.sc[p] << 23);  // 2^(e8m0 - 127)
-      const U4a8 x = w.nope[p];
+      const V4a8 x = w.nope[p];
       *reinterpret_cast<uint4*>(sKV + off) =
           make_uint4(cvt2_e4m3_bf16<false>(x.x, sc), cvt2_e4m3_bf16<true>(x.x, sc),
                      cvt2_e4m3_bf16<false>(x.y, sc), cvt2_e4m3_bf16<true>(x.y, sc));
@@ -335,10 +341,8 @@ __device__ __forceinline__ void attn_role(const AttnArgs& a, Smem<FMT>& sm) {
           make_uint4(cvt2_e4m3_bf16<false>(x.z, sc), cvt2_e4m3_bf16<true>(x.z, sc),
                      cvt2_e4m3_bf16<false>(x.w, sc), cvt2_e4m3_bf16<true>(x.w, sc));
     };
-    auto load_rope = [&](int at) -> U4a8 {
-      return *reinterpret_cast<const U4a8*>((uintptr_t)(sm.row[at + (ln >> 3)] + kANope + 16 * (ln & 7)));
-    };
-    auto store_rope = [&](int j, const U4a8& x) {  // then zeros for the rows past the list
+    auto load_rope = [&](int at) -> V4a8 { return ld_global<V4a8>(sm.row[at + (ln >> 3)] + kANope + 16 * (ln & 7)); };
+    auto store_rope = [&](int j, const V4a8& x) {  // then zeros for the rows past the list
       const int t = 8 * wo + (ln >> 3);
       uint8_t* tile = sKV + (j & (kRing - 1)) * kTile;
       *reinterpret_cast<uint4*>(tile + t * 1024 + (((56 + (ln & 7)) ^ sw(t)) << 4)) = make_uint4(x.x, x.y, x.z, x.w);
