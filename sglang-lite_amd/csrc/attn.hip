@@ -51,59 +51,11 @@
 // (640 indices, -1 where a token has fewer rows) 320 -> 182 us.  The roles
 // without the MFMAs between reads and gathers (each fragment read waited for
 // by itself): 1.3 us a block.
-#include "sgl_common.h"
+#include "sgl_attn.h"
 #include "sgl_numeric.h"
-#include "sgl_rules.h"
 
 namespace sgl {
 namespace {
-
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-typedef short v4s __attribute__((ext_vector_type(4)));
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef v4s __attribute__((address_space(3))) lds_v4s;
-
-constexpr int kD = 512;     // head dim: 448 latent + 64 rope
-constexpr int kBlk = 64;    // indices a split is cut by
-constexpr int kHG = 64;     // heads per workgroup
-constexpr int kARow = 584, kAData = 576, kANope = 448;
-constexpr float kLog2e = 1.4426950408889634f;
-
-struct AttnArgs {
-  const uint16_t* q;   // [B, M, Hh, 512] bf16
-  const uint8_t* kv;   // per batch element: bf16 [n, ld] | layout A [n, 584] | layout A pages
-  int64_t n;           // rows per batch element
-  int64_t kv_bstride;  // bytes between batch elements
-  int64_t ld;          // bf16 rows: elements per row
-  int page;            // footer pages: rows per page
-  int page_shift;      // log2(page) when page is a power of two, else -1
-  const float* sink;   // [Hh]
-  const int32_t* idx;  // [B, M, K]
-  int64_t M, K;
-  int Hh;
-  float scale;
-  uint16_t* o;         // [B, M, Hh, 512] bf16
-  int nsplit;          // > 1: the K rows are split over workgroups, partials to ws
-  int bps;             // 64-row blocks per split
-  float* ws_acc;       // [B, M, nsplit, Hh, 512] unnormalised outputs
-  float* ws_ml;        // [B, M, nsplit, Hh, 2] running max (log2 units) and sum
-};
-
-// Row-major tile: token t, 16-byte chunk c (8 dims) at t*1024 + ((c ^ sw(t)) << 4).
-// sw rotates the token's low four bits, which keeps conflict-free both the
-// S^T fragment reads (16 B of one chunk from 16 consecutive tokens) and the
-// transpose reads (8 B of 4 consecutive chunks from 4 consecutive tokens).
-__device__ __forceinline__ uint32_t sw(int t) { return (uint32_t)(((t & 3) << 2) | ((t >> 2) & 3)); }
-
-__device__ __forceinline__ v4s lds_tr16(const uint8_t* base, uint32_t off) {
-  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(base + off));
-}
-
-template <bool HI>
-__device__ __forceinline__ uint32_t cvt2_e4m3_bf16(uint32_t w, float sc) {
-  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, sc, HI));
-}
 
 // 16 bytes at an 8-byte aligned address (layout A rows)
 typedef uint32_t V4a8 __attribute__((ext_vector_type(4), aligned(8)));
@@ -767,7 +719,7 @@ __global__ __launch_bounds__(256) void sparse_attn_combine_kernel(const AttnArgs
 
 extern "C" size_t sgl_sparse_attn_workspace_size(int64_t B, int64_t M, int Hh, int64_t K) {
   if (B <= 0 || M <= 0 || Hh <= 0 || K <= 0) return 0;
-  const int ns = sgl::attn_splits(B * M, Hh, K, sgl::device_cu_count());
+  const int ns = sgl::attn_plan(B * M, Hh, K, sgl::device_cu_count()).nsplit;
   if (ns == 1) return 0;
   return (size_t)(B * M * ns * Hh) * (sgl::kD + 2) * 4;
 }
@@ -808,7 +760,8 @@ extern "C" int sgl_sparse_attn(const void* q, int64_t B, int64_t M, int Hh, cons
   a.Hh = Hh;
   a.scale = softmax_scale;
   a.o = (uint16_t*)o;
-  a.nsplit = sgl::attn_splits(B * M, Hh, K, sgl::device_cu_count());
+  const sgl::AttnPlan plan = sgl::attn_plan(B * M, Hh, K, sgl::device_cu_count());
+  a.nsplit = plan.nsplit;
   const int64_t nblk = (K + sgl::kBlk - 1) / sgl::kBlk;
   a.bps = (int)((nblk + a.nsplit - 1) / a.nsplit);
   a.ws_acc = nullptr;
@@ -833,7 +786,9 @@ extern "C" int sgl_sparse_attn(const void* q, int64_t B, int64_t M, int Hh, cons
     else                                                                \
       sgl::sparse_attn_kernel<FMT, 2><<<grid, 512, 0, st>>>(a);         \
   } while (0)
-  if (kv_format == SGL_ATTN_KV_BF16)
+  if (plan.few)
+    sgl::launch_sparse_attn_few(a, kv_format, grid, st);
+  else if (kv_format == SGL_ATTN_KV_BF16)
     SGL_ATTN(SGL_ATTN_KV_BF16);
   else if (kv_format == SGL_ATTN_KV_A)
     SGL_ATTN(SGL_ATTN_KV_A);

@@ -46,37 +46,56 @@ SGL_RULE AttnMerge attn_merge_at(uint32_t wg, uint32_t wave, uint32_t queries, u
   return {w / heads, w % heads};
 }
 
-// ---- sparse attention: the workgroups (splits) that share a query's K
-// indices, cut in 64s: at most one a CU, at most kAttnMaxSplits.  A function of
-// the shape alone and not of the cache's format, so that the packed cache gives
-// bit for bit what its dequantized rows give.
+// ---- sparse attention: the kernel, and the workgroups (splits) that share a
+// query's K indices, cut in 64s: at most one a CU, at most kAttnMaxSplits.  A
+// function of the shape alone and not of the cache's format, so that the packed
+// cache gives bit for bit what its dequantized rows give.
 //
 // A split shortens the serial chain of blocks but writes fp32 partials (128 KB
-// per 64 heads) that a merge reads back.  The cheapest by these costs, in
+// per 64 heads) that a merge reads back; attn_few.hip (at most 64 heads) starts
+// sooner than attn.hip but is slower a block.  The cheapest by these costs, in
 // 1/100 us, fitted to 1 ... 256 queries x 64 ... 2048 indices x 1 ... 128 heads,
-// bf16 rows and packed pages, every number of splits:
-//   a block of 64 indices: 250;
+// bf16 rows and packed pages, both kernels, every number of splits:
+//   a block of 64 indices: 250 (attn.hip, whose own blocks are 32 rows: at most
+//     32 indices 125);
+//   attn_few.hip against attn.hip: 75 a block more, and to start 285 - 3.6 heads
+//     less (at most 32 heads) or 150 - 2.4 (heads - 32) less;
 //   a merge: 140 and 31 a split, up to 88 more with the heads, and for each
 //     partial of 64 heads 4.5 where the merge follows its splits (a multiple of
 //     eight queries), else 7.2, at most 990.
-// (64 heads, packed pages, us: 32 / 33 queries x 128 indices, one split / two
+// (Packed pages, us.  64 heads: 32 / 33 queries x 128 indices, one split / two
 // 15.2 / 17.4 and 15.1 / 20.7; 32 x 384, one / three 25.3 / 20.8; 32 x 640, one
 // / five 35.6 / 23.5; 33 x 2048, seven 36.7, eight, which are 264 workgroups,
-// 52.6.)
+// 52.6.  256 queries, few / attn.hip: 8 heads x 64 indices 9.3 / 12.2, x 192
+// 16.1 / 17.0, x 640 38.7 / 36.9; 32 heads 12.3 / 14.1, 19.1 / 18.9, 41.3 /
+// 38.6; one query x 8 heads x 256, four splits 10.8 / 13.5, x 32 heads x 1 index
+// 9.2 / 8.5.)
 constexpr int kAttnMaxSplits = 8;
-SGL_RULE int attn_splits(int64_t queries, int heads, int64_t K, int cus) {
+struct AttnPlan {
+  bool few;  // attn_few.hip
+  int nsplit;
+};
+SGL_RULE AttnPlan attn_plan(int64_t queries, int heads, int64_t K, int cus) {
   const int64_t blocks = (K + 63) / 64, wgs = queries * ((heads + 63) / 64);
   const int64_t h64 = heads < 64 ? heads : 64;
-  int best = 1;
-  int64_t best_cost = blocks * 250;
-  for (int64_t want = 2; want <= kAttnMaxSplits && want <= blocks && want * wgs <= cus; ++want) {
-    const int64_t bps = (blocks + want - 1) / want, ns = (blocks + bps - 1) / bps;  // no empty split
-    int64_t parts = queries * ns * heads * (queries % 8 == 0 ? 45 : 72) / 640;
-    if (queries % 8 != 0 && parts > 990) parts = 990;
-    const int64_t cost = bps * 250 + 140 + 31 * ns + 88 * h64 / 64 + parts;
-    if (cost < best_cost) {
-      best_cost = cost;
-      best = (int)ns;
+  AttnPlan best = {false, 1};
+  int64_t best_cost = K <= 32 ? 125 : blocks * 250;
+  for (int kernel = 0; kernel < (heads <= 64 ? 2 : 1); ++kernel) {
+    const bool few = kernel == 1;
+    const int64_t start = !few ? 0 : heads <= 32 ? 285 - 36 * heads / 10 : 150 - 24 * (heads - 32) / 10;
+    for (int64_t want = 1; want <= kAttnMaxSplits && (want == 1 || (want <= blocks && want * wgs <= cus)); ++want) {
+      const int64_t bps = (blocks + want - 1) / want;
+      const int64_t ns = bps > 0 ? (blocks + bps - 1) / bps : 1;  // no empty split
+      int64_t cost = (!few && K <= 32 ? 125 : bps * (few ? 325 : 250)) - start;
+      if (ns > 1) {
+        int64_t parts = queries * ns * heads * (queries % 8 == 0 ? 45 : 72) / 640;
+        if (queries % 8 != 0 && parts > 990) parts = 990;
+        cost += 140 + 31 * ns + 88 * h64 / 64 + parts;
+      }
+      if (cost < best_cost) {
+        best_cost = cost;
+        best = {few, (int)ns};
+      }
     }
   }
   return best;

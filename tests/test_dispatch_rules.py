@@ -22,7 +22,8 @@ void merge_at(uint32_t wg, uint32_t wave, uint32_t queries, uint32_t M, uint32_t
   out[0] = m.query;
   out[1] = m.head;
 }
-int splits(int64_t queries, int heads, int64_t K, int cus) { return attn_splits(queries, heads, K, cus); }
+int splits(int64_t queries, int heads, int64_t K, int cus) { return attn_plan(queries, heads, K, cus).nsplit; }
+int few(int64_t queries, int heads, int64_t K, int cus) { return attn_plan(queries, heads, K, cus).few; }
 }
 """
 
@@ -62,7 +63,8 @@ def test_attention_merge_covers_and_follows_the_splits(rules, B, M, heads):
 
 @pytest.mark.parametrize("cus", [256, 64, 1])
 def test_attention_splits_fit_the_device(rules, cus):
-    """At most a workgroup per CU once a query is split, none of them empty."""
+    """At most a workgroup per CU once a query is split, none of them empty; the
+    few-head kernel for at most 64 heads."""
     i64 = ctypes.c_int64
     for queries in (1, 7, 8, 32, 33, 100, 128, 129, 256, 5000):
         for heads in (1, 8, 64, 65, 128):
@@ -70,8 +72,19 @@ def test_attention_splits_fit_the_device(rules, cus):
                 ns = rules.splits(i64(queries), heads, i64(K), cus)
                 blocks = -(-K // 64)
                 assert 1 <= ns <= 8
+                assert heads <= 64 or not rules.few(i64(queries), heads, i64(K), cus)
                 if ns > 1:
                     assert ns * queries * -(-heads // 64) <= cus
                     assert ns <= blocks and (ns - 1) * -(-blocks // ns) < blocks
     assert rules.splits(i64(32), 64, i64(640), 256) == 5
     assert rules.splits(i64(33), 64, i64(2048), 256) == 7
+
+
+@pytest.mark.parametrize("queries,heads,K,few", [
+    (1, 8, 64, 1), (1, 8, 256, 1), (32, 16, 256, 1), (16, 32, 192, 1), (1, 33, 64, 1), (256, 8, 128, 1),
+    (1, 64, 640, 0), (32, 64, 640, 0), (256, 32, 640, 0), (2048, 64, 640, 0), (2048, 8, 640, 0), (1, 128, 64, 0),
+    (1, 8, 1, 1), (1, 48, 1, 0), (64, 32, 32, 0), (64, 32, 33, 1),
+])
+def test_attention_kernel_by_chain(rules, queries, heads, K, few):
+    """Short chains of few heads take the kernel that starts sooner."""
+    assert rules.few(ctypes.c_int64(queries), heads, ctypes.c_int64(K), 256) == few

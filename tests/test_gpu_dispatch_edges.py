@@ -321,3 +321,24 @@ def test_sparse_attn_row_lists_by_valid_rows(gpu, valid, K):
     for s in (0, S - 1):
         ref = OA.sparse_attn_exact(q[:, s:s + 1], rows, sink, idx[:, s:s + 1], 512 ** -0.5)
         assert_gemm_close(got[:, s:s + 1], ref, f"valid={valid} query {s}")
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "rows", "pages"])
+@pytest.mark.parametrize("H,K", [(1, 1), (8, 63), (8, 64), (8, 65), (8, 256), (16, 300), (31, 128), (32, 130),
+                                 (33, 64), (40, 100), (63, 64), (64, 1)])
+def test_sparse_attn_short_chains(gpu, H, K, fmt):
+    """The kernel of few heads and short selections (one to a few blocks, split
+    or not, both sides of its 32 heads), masked entries among the rows, a query
+    with none."""
+    rng = np.random.default_rng(H * 1000 + K)
+    print(f"attn short H={H} K={K} {fmt}", flush=True)
+    for B, S in ((1, 2), (3, 1), (2, 64)):
+        n = 70
+        q, kv = bf16_values(rng, (B, S, H, 512)), bf16_values(rng, (B, n, 512))
+        sink = (rng.standard_normal(H) * 2).astype(np.float32)
+        idx = rng.integers(0, n, (B, S, K)).astype(np.int32)
+        idx[rng.random(idx.shape) < 0.2] = -1
+        idx[0, 0] = -1
+        got, rows = _attn(gpu, q, kv, sink, idx, 512 ** -0.5, fmt)
+        assert_gemm_close(got, OA.sparse_attn_blocked(q, rows, sink, idx, 512 ** -0.5), f"H={H} K={K} {fmt} {B}x{S}")
+        assert np.all(got[0, 0] == 0)
