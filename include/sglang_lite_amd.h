@@ -198,10 +198,11 @@ int sgl_mfma_mix_threads(void);
  * Shapes for which sgl_fp8_gemm_workspace_size is non-zero (16 < M <= 64
  * with N % 128 == 0) need a workspace (16-byte aligned, at least that many
  * bytes; a smaller one is SGL_ERR_WORKSPACE): where the K range is split over
- * workgroups it holds the fp32 partials; most of these shapes split K inside
+ * workgroups it holds the fp32 partials; the others split K inside
  * a workgroup instead and leave it untouched.  Which it is depends on the
- * shape and the kinds of scales alone, so eager and graph-captured calls sum
- * in the same order.  Calls that overlap in time need workspaces of their own.
+ * shape (and the device's CU count) alone, so eager and graph-captured calls
+ * sum in the same order.  Calls that overlap in time need workspaces of their
+ * own.
  * Replaces deepseek_infer/kernel.py:257-273 fp8_gemm (kernel :203-254) and the
  * call-site adapter engine/v4_deep_gemm.py:169-218 fp4_gemm_nt (whose
  * workspace-free call the reference's adapter allocates with torch at

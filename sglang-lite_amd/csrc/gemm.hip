@@ -41,6 +41,7 @@
 #include "sgl_dense_mid.h"
 #include "sgl_gemm.h"
 #include "sgl_numeric.h"
+#include "sgl_rules.h"
 
 namespace sgl {
 namespace {
@@ -3000,8 +3001,8 @@ int launch_skinny(GemmArgs& a, hipStream_t stream) {
 // us + 4 us, against 22.6 us for the skinny kernel.  A last-workgroup sum in
 // place of the second launch costs three dependent trips to device-coherent
 // memory, about 3 us.)  The tiles that split K inside a workgroup need no
-// partials and take the shape wherever they cover the CUs (11.8 us there with
-// e8m0 scales, split-K 14.7); this is what is left: few tiles, or fp32 scales.
+// partials and take the shapes of short K or many tiles (dense_k_groups); this
+// is what is left.
 namespace splitk {
 constexpr int NW = 8, NT = 64 * NW, BN = 16 * NW, KSMAX = 8, SMAX = 16, TMMAX = 4;
 }  // namespace splitk
@@ -3273,14 +3274,9 @@ int try_splitk(GemmArgs& a, hipStream_t stream) {
               (long long)a.M, (long long)a.N, (long long)a.K, S, need, a.ws ? a.ws_bytes : (size_t)0);
     return SGL_ERR_WORKSPACE;
   }
-  // K groups inside a workgroup where their tiles cover enough CUs: no
-  // partials, no second launch (e8m0 scales, us split / K groups: N = 4096,
-  // K = 7168, M = 32 / 64 12.6 / 12.0 and 14.7 / 11.8; K = 2048 8.9 / 6.3 and
-  // 11.8 / 6.2; N = 1536, K = 4096, M = 64, 48 tiles, 10.5 / 8.4; but M = 32, 24
-  // tiles, 8.2 / 8.4, and N = 512, K = 7168, M = 64, 16 tiles, 9.3 / 10.8; at
-  // K = 1024 6.1 / 4.4 even with 16)
-  const bool scaled = a.sa_e8m0 && a.sb_e8m0;  // (fp32 scales at M = 24, N = 4096, K = 7168: 11.9 / 12.4)
-  if (a.K < 4096 || ((scaled || a.M > 32) && ceil_div(a.M, (int64_t)32) * ceil_div(a.N, (int64_t)64) > 24)) {
+  // K groups inside a workgroup where they are the faster: no partials, no
+  // second launch
+  if (dense_k_groups(a.M, a.N, a.K, true)) {
     const int rc = launch_dense_mid(a, stream);
     if (rc != kNoMid) return rc;
   }
@@ -3557,7 +3553,8 @@ int launch_gemm(int kind, GemmArgs& a, int64_t rows_hint, hipStream_t stream) {
     case KIND_DENSE: {
       const int rc = SGL_SPLITK ? try_splitk(a, stream) : kNoSplit;
       if (rc != kNoSplit) return rc;
-      if (a.M > 16) {  // (at M = 16 the skinny kernel's 9.5 us against 12.2)
+      // (at M = 16 the skinny kernel's 9.5 us against 12.2)
+      if (a.M > 16 && dense_k_groups(a.M, a.N, a.K, false)) {
         const int rm = launch_dense_mid(a, stream);
         if (rm != kNoMid) return rm;
       }

@@ -101,4 +101,23 @@ SGL_RULE AttnPlan attn_plan(int64_t queries, int heads, int64_t K, int cus) {
   return best;
 }
 
+// ---- dense FP8 GEMM, 16 < M <= 64: the tiles that split K inside a workgroup
+// (dense_mid.hip) against the split over workgroups (`splits`: the shape has
+// one) or else the skinny kernel.  A workgroup of those tiles walks all of K,
+// so they win where K is short or their tiles are many, at every format of the
+// scales.  N = 512 ... 7168, K = 1024 ... 8192, the weight out of memory / out of
+// the last-level cache, split over workgroups against K groups, us:
+// N = 4096: K = 2048, M = 32 -15 / -24 %, K = 4096 -6 / -18, K = 7168 +24 / -3,
+// M = 64, K = 7168 +6 / -18; N = 2048, M = 64, K = 4096 -7 / -28, K = 5120 +19 /
+// -15; N = 1024, K = 2048, M = 32 / 64 +7 / -11 out of memory, K = 4096 +40 / +17;
+// N = 512, K = 7168 +87 / +58.  The line keeps every shape within 8 % of the
+// better one out of memory, and gives up no gain there above 7 %.  Against the
+// skinny kernel, M = 17 ... 32: N = 3600, K = 2048 +40 %, 4112 -2 ... -5, 7168 -6
+// ... -20 (but K = 128 4.0 us / 4.6); from M = 33 -1 ... -56 % at every N and K.
+SGL_RULE bool dense_k_groups(int64_t M, int64_t N, int64_t K, bool splits) {
+  if (M > 64) return true;
+  const int64_t tiles = (M + 31) / 32 * ((N + 63) / 64);
+  return splits ? K <= 1024 || K <= 48 * tiles : M > 32 || (tiles >= 64 && K > 128);
+}
+
 }  // namespace sgl

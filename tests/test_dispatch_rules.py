@@ -24,6 +24,7 @@ void merge_at(uint32_t wg, uint32_t wave, uint32_t queries, uint32_t M, uint32_t
 }
 int splits(int64_t queries, int heads, int64_t K, int cus) { return attn_plan(queries, heads, K, cus).nsplit; }
 int few(int64_t queries, int heads, int64_t K, int cus) { return attn_plan(queries, heads, K, cus).few; }
+int k_groups(int64_t M, int64_t N, int64_t K, int splits) { return dense_k_groups(M, N, K, splits); }
 }
 """
 
@@ -88,3 +89,16 @@ def test_attention_splits_fit_the_device(rules, cus):
 def test_attention_kernel_by_chain(rules, queries, heads, K, few):
     """Short chains of few heads take the kernel that starts sooner."""
     assert rules.few(ctypes.c_int64(queries), heads, ctypes.c_int64(K), 256) == few
+
+
+@pytest.mark.parametrize("M,N,K,splits,groups", [
+    (17, 512, 3072, 1, 0), (32, 1024, 4096, 1, 0), (33, 1024, 7168, 1, 0), (32, 4096, 7168, 1, 0),
+    (64, 1536, 8192, 1, 0), (32, 512, 1024, 1, 1), (32, 4096, 2048, 1, 1), (64, 4096, 4096, 1, 1),
+    (17, 576, 7168, 0, 0), (32, 2112, 512, 0, 0), (33, 576, 7168, 0, 1), (32, 7168, 8192, 0, 1),
+    (32, 4096, 128, 0, 0), (65, 512, 7168, 0, 1), (4096, 512, 7168, 0, 1),
+])
+def test_dense_k_groups_where_they_win(rules, M, N, K, splits, groups):
+    """Long K over few tiles stays split over workgroups, narrow products of at
+    most 32 rows on the skinny kernel."""
+    i64 = ctypes.c_int64
+    assert rules.k_groups(i64(M), i64(N), i64(K), splits) == groups
