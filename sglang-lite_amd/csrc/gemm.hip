@@ -3448,24 +3448,16 @@ inline bool rb_fp4_ok(const GemmArgs& a) {
          aligned(a.sa, 16);
 }
 
-// Rows per expert, on average, from which the grouped GEMMs take 128-row
-// tiles.  Below, the 32-row decode tiles stream each expert's weights once
-// per tile; above, most experts fill a second 32-row tile and the weights are
-// streamed (through L2) again for it, while a 128-row tile takes them once.
-// Layer of H = 4096, I = 2048, top-8, 32-row / 128-row tiles, uniform and
-// skewed load, bit-identical outputs:
-//   FP8 (pipelined kernel) E = 256: 26 rows 1187 / 1249 and 1350 / 1287 us,
-//     29 rows 1285 / 1256 and 1442 / 1291, 59 rows 1986 / 1364 and 2060 / 1465;
-//     E = 64: 28 rows 343 / 361 and 370 / 359, 37 rows 395 / 367 and 402 / 364
-//   FP4 E = 256: 29 rows 888 / 982 and 1008 / 1045, 38 rows 1142 / 1007 and
-//     1134 / 1079, 59 rows 1406 / 1079 and 1461 / 1205; E = 64: 37 rows
-//     338 / 298 and 317 / 338, 50 rows 380 / 307 and 380 / 345
-constexpr int64_t kPipeRows = 29;
-constexpr int64_t kFp4BigRows = 38;
+// Whether a grouped launch takes 128-row tiles (columns of a tile: 128 of gate
+// and of up, or 256)
+bool tall_tiles(int kind, const GemmArgs& a, int64_t rows_hint) {
+  const int64_t cols = ceil_div(a.N, (int64_t)(kind == KIND_GATE_UP ? 128 : 256));
+  return moe_tall_tiles(a.wfmt == WF_FP4, rows_hint, std::max(a.E, 1) * cols, device_cu_count());
+}
 
 template <bool SAHW>
 int launch_fp4(int kind, GemmArgs& a, int64_t rows_hint, hipStream_t stream) {
-  const bool big = rows_hint >= kFp4BigRows;
+  const bool big = tall_tiles(kind, a, rows_hint);
   switch (kind) {
     case KIND_DENSE:
       if (a.M <= kSkinnyMaxM) {
@@ -3518,7 +3510,7 @@ int launch_gemm(int kind, GemmArgs& a, int64_t rows_hint, hipStream_t stream) {
   const bool big = rows_hint >= 64;
   // the pipelined prefill kernel: K in [512, 8192] (at least four stages; the
   // tile's weight scales fit its LDS table) and fp32 weight scales
-  const bool pipe_ok = SGL_PIPE && rows_hint >= kPipeRows && a.K >= 512 &&
+  const bool pipe_ok = SGL_PIPE && tall_tiles(kind, a, rows_hint) && a.K >= 512 &&
                        a.K <= 128 * pipe::kMaxKBp && !a.sb_e8m0;
   // both scales powers of two: the pipelined kernel applies them in the MFMA
   // (other kernels promote in fp32, exact for such scales too)

@@ -111,13 +111,39 @@ SGL_RULE AttnPlan attn_plan(int64_t queries, int heads, int64_t K, int cus) {
 // M = 64, K = 7168 +6 / -18; N = 2048, M = 64, K = 4096 -7 / -28, K = 5120 +19 /
 // -15; N = 1024, K = 2048, M = 32 / 64 +7 / -11 out of memory, K = 4096 +40 / +17;
 // N = 512, K = 7168 +87 / +58.  The line keeps every shape within 8 % of the
-// better one out of memory, and gives up no gain there above 7 %.  Against the
+// better one out of memory, and gives up no gain there above 12 %.  Against the
 // skinny kernel, M = 17 ... 32: N = 3600, K = 2048 +40 %, 4112 -2 ... -5, 7168 -6
 // ... -20 (but K = 128 4.0 us / 4.6); from M = 33 -1 ... -56 % at every N and K.
 SGL_RULE bool dense_k_groups(int64_t M, int64_t N, int64_t K, bool splits) {
   if (M > 64) return true;
   const int64_t tiles = (M + 31) / 32 * ((N + 63) / 64);
   return splits ? K <= 1024 || K <= 48 * tiles : M > 32 || (tiles >= 64 && K > 128);
+}
+
+// ---- grouped GEMMs of the MoE layer: 128-row tiles against the 32-row decode
+// tiles, by the rows of an expert on average and the 128-row tiles there are
+// when every expert has one.  The 32-row tiles stream each expert's weights
+// once per tile (through L2); above 32 rows most experts fill a second one,
+// while a 128-row tile takes the weights once.  But its tiles have to fill the
+// CUs: over one or two rounds of them the last, partly filled round costs what
+// the weights save.  From 64 rows the 128-row tiles always.
+// Layer, 32-row / 128-row tiles in us, uniform and skewed load (`rounds`: tiles
+// over CUs), bit-identical outputs:
+//   FP8, 16 rounds (H = 4096, I = 2048, E = 256): 26 rows 1187 / 1249 and 1350 /
+//     1287, 29 rows 1285 / 1256 and 1442 / 1291, 59 rows 1986 / 1364 and 2060 /
+//     1465; 4 (E = 64): 29 rows 352 / 371 and 370 / 362, 36 rows 401 / 375 and 415 /
+//     370; 2 (H = 2048, I = 1024, E = 64): 29 rows 114 / 140 and 130 / 138, 36 rows
+//     135 / 143 and 135 / 140, 45 rows 157 / 146 and 157 / 143; 1 (E = 16): 29 rows
+//     117 / 157 and 118 / 161, 45 rows 150 / 154 and 152 / 152, 58 rows 155 / 159
+//     and 157 / 150; half a round (E = 8): 32 rows +6 and +8 %, 36 rows -29 and -26 %
+//   FP4, 16: 29 rows 888 / 982 and 1008 / 1045, 38 rows 1142 / 1007 and 1134 /
+//     1079; 4: 38 rows 346 / 306 and 324 / 340, 42 rows 350 / 305 and 349 / 342; 2
+//     (E = 32): 46 rows -11 and +5 %, 52 rows -18 and -5 %; 1: 50 rows 138 / 112 and
+//     139 / 154, 60 rows 169 / 122 and 169 / 157.
+SGL_RULE bool moe_tall_tiles(bool fp4, int64_t rows, int64_t tiles, int64_t cus) {
+  if (rows >= 64) return true;
+  if (fp4) return (rows - 36) * tiles >= 28 * cus;
+  return (rows - 29) * tiles >= 20 * cus || (rows > 32 && 2 * tiles <= cus);
 }
 
 }  // namespace sgl

@@ -24,6 +24,7 @@ void merge_at(uint32_t wg, uint32_t wave, uint32_t queries, uint32_t M, uint32_t
 }
 int splits(int64_t queries, int heads, int64_t K, int cus) { return attn_plan(queries, heads, K, cus).nsplit; }
 int few(int64_t queries, int heads, int64_t K, int cus) { return attn_plan(queries, heads, K, cus).few; }
+int tall(int fp4, int64_t rows, int64_t tiles, int64_t cus) { return moe_tall_tiles(fp4, rows, tiles, cus); }
 int k_groups(int64_t M, int64_t N, int64_t K, int splits) { return dense_k_groups(M, N, K, splits); }
 }
 """
@@ -102,3 +103,15 @@ def test_dense_k_groups_where_they_win(rules, M, N, K, splits, groups):
     most 32 rows on the skinny kernel."""
     i64 = ctypes.c_int64
     assert rules.k_groups(i64(M), i64(N), i64(K), splits) == groups
+
+
+@pytest.mark.parametrize("fp4,rows,tiles,tall", [
+    (0, 31, 4096, 1), (0, 29, 4096, 0), (0, 32, 1024, 0), (0, 36, 1024, 1), (0, 36, 512, 0), (0, 40, 512, 1),
+    (0, 40, 256, 0), (0, 64, 256, 1), (0, 32, 128, 0), (0, 33, 128, 1), (0, 64, 1, 1),
+    (1, 38, 4096, 1), (1, 37, 4096, 0), (1, 38, 1024, 0), (1, 43, 1024, 1), (1, 46, 512, 0), (1, 52, 512, 1),
+    (1, 58, 256, 0), (1, 64, 256, 1),
+])
+def test_moe_tiles_need_rounds(rules, fp4, rows, tiles, tall):
+    """128-row tiles below 64 rows an expert only where they fill the CUs often enough."""
+    i64 = ctypes.c_int64
+    assert rules.tall(fp4, i64(rows), i64(tiles), i64(256)) == tall

@@ -17,11 +17,12 @@ from test_gpu_moe import table_from
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("fp4,T", [(False, 56), (False, 58), (True, 74), (True, 76)])
+@pytest.mark.parametrize("fp4,T", [(False, 56), (False, 58), (True, 74), (True, 76), (False, 64), (False, 66),
+                                   (True, 126), (True, 128)])
 def test_moe_tile_rule(gpu, fp4, T):
     """Average rows per expert just below and at the 128-row tiles' threshold
-    (FP8 29, FP4 38), with uneven groups (an expert with no row, one with one,
-    the last with the rest)."""
+    (with these few tiles FP8 33, FP4 64), with uneven groups (an expert with
+    no row, one with one, the last with the rest)."""
     from sglang_lite_amd import moe as M
 
     rng = np.random.default_rng(T + fp4)
