@@ -347,8 +347,9 @@ size_t sgl_moe_workspace_size(int64_t T, int64_t H, int64_t I, int E, int k, int
 /* Whole routed+shared MoE layer from bf16 x [T, H] and a precomputed top-k
  * (ids int32 [T, k], weights fp32 [T, k]): act quant -> permute -> gate/up
  * -> down -> combine, y bf16 [T, H]; routed experts in expert_format.
- * The smallest batches (FP4 T*k <= 24, FP8 T = 1 or T*k <= 8) run gate/up and
- * down without a permute or combine; the same rounding points and workspace.
+ * The smallest batches (FP4 T*k <= 24, FP8 T = 1 or T*k <= 8, while the picked
+ * experts are few or small enough) run gate/up and down without a permute or
+ * combine; the same rounding points and workspace.
  * Replaces engine/v4_moe_fast.py:79-106 _moe_forward_activated_only after
  * the gate.  Every launch goes to `stream`. */
 int sgl_moe_forward(const void* x, int64_t T, int64_t H, int64_t I, int E, int k,

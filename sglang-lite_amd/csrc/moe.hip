@@ -1371,7 +1371,7 @@ int sgl_moe_forward(const void* x, int64_t T, int64_t H, int64_t I, int E, int k
     return rc;
   hipStream_t st = (hipStream_t)stream;
   const bool fp4 = sgl::fp4_experts(expert_format);
-  if (sgl::small_moe_ok(T, H, I, k, has_shared, fp4)) {
+  if (sgl::small_moe_ok(T, H, I, k, has_shared, fp4, sgl::device_cu_count())) {
     sgl::SmallMoeArgs a = {};
     a.xq = w.xq;
     a.xs = w.xs;

@@ -39,7 +39,7 @@ namespace {
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-constexpr int kMaxSlots = 64;  // T k: one lane a slot
+constexpr int kMaxSlots = kSmallMoeSlots;
 
 // One 128-deep K block of a row in MFMA lane order, lane group g: fp8 bytes
 // [32 g, +32); the fp8 side of a product with fp4 bytes [16 g, +16) and
@@ -254,16 +254,8 @@ void small_gate_up_kernel(const SmallMoeArgs a) {
 }
 
 // --------------------------------------------------------------------- down
-constexpr int kDnWaves = 16;
-constexpr int kDnLds = 157 * 1024;
-
-// LDS of R = T (k + shared) rows: h as e4m3 with its scales, and the partial
-// outputs of each line of K; the rest holds weights, 2 KB lines of each
-// wavefront.
-__host__ __device__ constexpr int64_t down_rows_bytes(int64_t R, int64_t I) { return R * (I + I / 32 + I / 2); }
-__host__ __device__ constexpr int down_slots(int64_t R, int64_t I) {
-  return (int)((kDnLds - down_rows_bytes(R, I)) / (kDnWaves * 2048));
-}
+constexpr int kDnWaves = kSmallDownWaves;
+constexpr int kDnLds = kSmallDownLds;  // (small_down_rows_bytes, then weights)
 
 struct DnTables {
   int id[kMaxSlots];         // the slots' experts
@@ -482,23 +474,11 @@ __global__ __launch_bounds__(64 * kDnWaves) void small_down_kernel(const SmallMo
 
 }  // namespace
 
-// The lines, H = 4096, I = 2048, grouped path / this one in us, E = 256 (64
-// within a few percent): FP4 experts T k = 8 (T = 1) 77.7 / 38.9, 16 (T = 2)
-// 82 / 67 and (T = 4) 94 / 63, 24 (T = 3) 110 / 87 and (T = 4) 123 / 86, above
-// which h leaves too little LDS for the weights; FP8, whose grouped launches
-// already are two, 8 (T = 1) 67 / 58 and (T = 2) 67 / 56, 12 (T = 2) 78 / 77 and
-// (T = 3) 72 / 72, 16 (T = 2) 91 / 96.
-bool small_moe_ok(int64_t T, int64_t H, int64_t I, int k, int has_shared, bool fp4) {
-  const int64_t R = T * (k + has_shared);
-  if (fp4 ? T * k > 24 : T > 1 && T * k > 8) return false;
-  return T * k <= kMaxSlots && I <= H && down_rows_bytes(R, I) <= kDnLds && down_slots(R, I) >= 2;
-}
-
 int launch_small_moe(const SmallMoeArgs& a, bool fp4, hipStream_t st) {
   const int64_t S = a.T * a.k, R = S + (a.has_shared ? a.T : 0);
   const unsigned gu = (unsigned)(S * (a.I / (fp4 ? 16 : 8)) + (a.has_shared ? a.I / 8 : 0));
   const unsigned dn = (unsigned)(a.H / 16);
-  const int slots = std::min(5, down_slots(R, a.I));
+  const int slots = std::min(5, small_down_slots(R, a.I));
   if (fp4) {
     small_gate_up_kernel<true><<<gu, 64 * kGuWaves, 0, st>>>(a);
     small_down_kernel<true><<<dn, 64 * kDnWaves, 0, st>>>(a, slots);

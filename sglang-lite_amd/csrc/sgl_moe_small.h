@@ -3,6 +3,7 @@
 #pragma once
 
 #include "sgl_common.h"
+#include "sgl_rules.h"
 
 namespace sgl {
 
@@ -21,10 +22,7 @@ struct SmallMoeArgs {
   uint16_t* y;   // bf16 [T, H]
 };
 
-// Whether a layer of these sizes takes this path: where it fits (h in the
-// workspace of the down projection's rows, I <= H, and its quantized copy in
-// the LDS of a CU) and is the faster one.
-bool small_moe_ok(int64_t T, int64_t H, int64_t I, int k, int has_shared, bool fp4);
+// (the sizes: small_moe_ok)
 int launch_small_moe(const SmallMoeArgs& args, bool fp4, hipStream_t stream);
 
 }  // namespace sgl

@@ -146,4 +146,42 @@ SGL_RULE bool moe_tall_tiles(bool fp4, int64_t rows, int64_t tiles, int64_t cus)
   return (rows - 29) * tiles >= 20 * cus || (rows > 32 && 2 * tiles <= cus);
 }
 
+// ---- MoE layer of the smallest batches: the two launches of moe_small.hip
+// against the grouped path, where they fit (h in the workspace of the down
+// projection's rows, and its quantized copy in the LDS of a CU) and are the
+// faster.  Layer, grouped / these in us, E = 256 (64 within a few percent;
+// tables with fragment copies 0 to 9 % more of the grouped path):
+//   FP4, H = 4096, I = 2048: T k = 1 (T = 1) 81 / 18, 8 (T = 1) 74 / 41, 16 82 / 68,
+//     24 (T = 3) 112 / 96, above which h leaves too little LDS for the weights;
+//     H = 7168: 8 91 / 65, 24 (T = 3) 153 / 148.  Without a shared expert the
+//     grouped path has two launches less: H = 4096, 12 53 / 49, 16 59 / 62; H =
+//     7168, 8 68 / 58, 16 88 / 106; H = 5120, I = 1536, 16 71 / 70, 24 83 / 92.
+//   FP8, whose grouped launches already are two and read at the memory's rate,
+//     win by the launches saved only while the experts' bytes are few: H = 4096,
+//     I = 2048, T = 1: k = 1 55 / 19, 8 64 / 57, 9 66 / 63, 12 76 / 79, 14 86 / 90;
+//     H = 7168, k = 4 75 / 57, 5 78 / 65, 8 89 / 92; H = 3072, I = 1536, k = 16
+//     62 / 66; H = 2048, I = 1024, k = 16 44 / 40.
+//     T = 1 again where the grouped gate/up needs a second round of workgroups:
+//     k = 16 at H = 4096 121 / 100, at 7168 167 / 162 (one round at H = 5120, I =
+//     1536 93 / 111).
+constexpr int kSmallMoeSlots = 64;  // T k: one lane a slot
+constexpr int kSmallDownWaves = 16;
+constexpr int kSmallDownLds = 157 * 1024;
+// LDS of R = T (k + shared) rows: h as e4m3 with its scales, and the partial
+// outputs of each line of K; the rest holds weights, 2 KB lines of each
+// wavefront.
+SGL_RULE int64_t small_down_rows_bytes(int64_t R, int64_t I) { return R * (I + I / 32 + I / 2); }
+SGL_RULE int small_down_slots(int64_t R, int64_t I) {
+  return (int)((kSmallDownLds - small_down_rows_bytes(R, I)) / (kSmallDownWaves * 2048));
+}
+SGL_RULE bool small_moe_ok(int64_t T, int64_t H, int64_t I, int k, int has_shared, bool fp4, int cus) {
+  const int64_t S = T * k, R = T * (k + has_shared);
+  if (S > (fp4 ? 24 : T > 1 ? 8 : kSmallMoeSlots)) return false;
+  if (fp4 && !has_shared && S * H * I > (int64_t)16 * 5120 * 1536) return false;
+  if (!fp4 && S * (H * I + (1 << 18)) > (int64_t)9 * (4096 * 2048 + (1 << 18)) &&
+      !(T == 1 && (k + has_shared) * (I / 128) > cus))
+    return false;
+  return I <= H && small_down_rows_bytes(R, I) <= kSmallDownLds && small_down_slots(R, I) >= 2;
+}
+
 }  // namespace sgl

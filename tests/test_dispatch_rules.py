@@ -24,6 +24,9 @@ void merge_at(uint32_t wg, uint32_t wave, uint32_t queries, uint32_t M, uint32_t
 }
 int splits(int64_t queries, int heads, int64_t K, int cus) { return attn_plan(queries, heads, K, cus).nsplit; }
 int few(int64_t queries, int heads, int64_t K, int cus) { return attn_plan(queries, heads, K, cus).few; }
+int small_moe(int64_t T, int64_t H, int64_t I, int k, int shared, int fp4) {
+  return small_moe_ok(T, H, I, k, shared, fp4, 256);
+}
 int tall(int fp4, int64_t rows, int64_t tiles, int64_t cus) { return moe_tall_tiles(fp4, rows, tiles, cus); }
 int k_groups(int64_t M, int64_t N, int64_t K, int splits) { return dense_k_groups(M, N, K, splits); }
 }
@@ -115,3 +118,24 @@ def test_moe_tiles_need_rounds(rules, fp4, rows, tiles, tall):
     """128-row tiles below 64 rows an expert only where they fill the CUs often enough."""
     i64 = ctypes.c_int64
     assert rules.tall(fp4, i64(rows), i64(tiles), i64(256)) == tall
+
+
+@pytest.mark.parametrize("fp4,T,H,I,k,small", [
+    (0, 1, 3072, 1536, 12, 1), (0, 1, 3072, 1536, 16, 0), (0, 1, 7168, 2048, 5, 1),
+    (0, 1, 4096, 2048, 8, 1), (0, 1, 4096, 2048, 9, 1), (0, 1, 4096, 2048, 12, 0), (0, 1, 4096, 2048, 14, 0),
+    (0, 1, 4096, 2048, 16, 1), (0, 1, 7168, 2048, 4, 1), (0, 1, 7168, 2048, 8, 0), (0, 2, 7168, 2048, 4, 0),
+    (0, 1, 7168, 2048, 16, 1), (0, 1, 5120, 1536, 12, 0), (0, 1, 5120, 1536, 16, 0), (0, 1, 2048, 1024, 16, 1),
+    (0, 2, 4096, 2048, 4, 1), (0, 2, 512, 512, 5, 0), (0, 1, 256, 384, 2, 0),
+    (1, 1, 4096, 2048, 16, 1), (1, 3, 4096, 2048, 8, 1), (1, 4, 4096, 2048, 8, 0), (1, 24, 4096, 2048, 1, 0),
+])
+def test_smallest_moe_batches_where_they_win(rules, fp4, T, H, I, k, small):
+    """FP8 layers leave the two-launch path where their experts' bytes outweigh the launches."""
+    i64 = ctypes.c_int64
+    assert rules.small_moe(i64(T), i64(H), i64(I), k, 1, fp4) == small
+
+
+@pytest.mark.parametrize("T,H,I,k,small", [(1, 4096, 2048, 8, 1), (1, 4096, 2048, 12, 1), (1, 4096, 2048, 16, 0),
+                                           (2, 7168, 2048, 8, 0), (3, 5120, 1536, 8, 0), (3, 3072, 1536, 8, 1)])
+def test_smallest_fp4_batches_without_a_shared_expert(rules, T, H, I, k, small):
+    i64 = ctypes.c_int64
+    assert rules.small_moe(i64(T), i64(H), i64(I), k, 0, 1) == small
