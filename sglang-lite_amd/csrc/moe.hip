@@ -13,6 +13,7 @@
 #include "sgl_gemm.h"
 #include "sgl_moe_small.h"
 #include "sgl_numeric.h"
+#include "sgl_rules.h"
 
 namespace sgl {
 namespace {
@@ -1245,35 +1246,36 @@ int sgl_moe_gate(const void* x, const void* w, int64_t T, int64_t H, int E, int 
   hipStream_t st = (hipStream_t)stream;
   const uint16_t* xb = (const uint16_t*)x;
   const uint16_t* wb = (const uint16_t*)w;
-  // T > 256 with H % 64 == 0: the LDS-staged kernels, the largest of their
-  // tiles that still gives about a workgroup per CU.  K split over the four
-  // wavefronts for the 32 x 32 tiles when H % 128 == 0 (H = 4096, E = 256
-  // projection: T = 512 13.0 -> 9.4 us); for the larger tiles two or four
-  // groups of four wavefronts, a 64-deep K block of the stage each, as the
-  // serial chain of a stage is walked half or a quarter as often (gate, one
-  // group or the four-way split / these: T = 2048 19.8 / 18.5 us, 3000 31.2 /
-  // 28.4, 3900 29.6 / 27.9, 4200 36.9 / 32.5, 8192 43.4 / 43.0 on a repeated
-  // x and 40.5 / 36.2 on a fresh one, 16384 87.6 / 89.7; H = 7168: T = 5000
-  // 80 / 58, 16384 122.3 / 121.7).  The choice between them is one round of
-  // tiles where there is one (T = 6000 in two rounds of 32 x 128 46 us, in one
-  // of 64 x 128 34; T = 3000 27.1 in 32 x 128 tiles, but two sums as long
-  // instead of four err by 2.7e-7 rather than 1.9e-7).  Decode-sized
-  // batches: the register-loaded kernel with 16 tokens x 16 experts per
-  // workgroup and 16 wavefronts with all their K steps in flight (many small
+  // T > 256 with H % 64 == 0: the LDS-staged kernels (router_tile).
+  // Decode-sized batches: the register-loaded kernel with 16 tokens x 16 experts
+  // per workgroup and 16 wavefronts with all their K steps in flight (many small
   // workgroups spread the weight read); it also serves H % 64 != 0 (64 x 64 or
   // 64 x 128 tiles).
-  auto tiles = [&](int64_t tt, int64_t te) { return sgl::ceil_div(T, tt) * sgl::ceil_div(E, te); };
-  if (T > 256 && H % 128 == 0 && tiles(32, 64) < 240) {
-    sgl::launch_router_ks<32, 32, 8>(xb, wb, T, (int)H, E, logits, st);
-  } else if (T > 256 && H % 64 == 0) {
-    if (tiles(32, 128) > 256)
-      sgl::launch_router_lds<64, 128, 3, 2>(xb, wb, T, (int)H, E, logits, st);
-    else if (tiles(32, 128) >= 240)
-      sgl::launch_router_lds<32, 128, 3, 2>(xb, wb, T, (int)H, E, logits, st);
-    else if (tiles(32, 64) >= 240)
-      sgl::launch_router_lds<32, 64, 3, 4>(xb, wb, T, (int)H, E, logits, st);
-    else
-      sgl::launch_router_lds<32, 32, 8>(xb, wb, T, (int)H, E, logits, st);
+  if (T > 256 && H % 64 == 0) {
+    const sgl::RouterTile t = sgl::router_tile(T, H, E);
+    const int h = (int)H;
+    if (t.tokens == 64) {
+      if (t.k == sgl::kGroups)
+        sgl::launch_router_lds<64, 128, 3, 2>(xb, wb, T, h, E, logits, st);
+      else
+        sgl::launch_router_lds<64, 128, 4>(xb, wb, T, h, E, logits, st);
+    } else if (t.experts == 128) {
+      if (t.k == sgl::kGroups)
+        sgl::launch_router_lds<32, 128, 3, 2>(xb, wb, T, h, E, logits, st);
+      else
+        sgl::launch_router_lds<32, 128, 4>(xb, wb, T, h, E, logits, st);
+    } else if (t.experts == 64) {
+      if (t.k == sgl::kGroups)
+        sgl::launch_router_lds<32, 64, 3, 4>(xb, wb, T, h, E, logits, st);
+      else if (t.k == sgl::kSplit4)
+        sgl::launch_router_ks<32, 64, 6>(xb, wb, T, h, E, logits, st);
+      else
+        sgl::launch_router_lds<32, 64, 6>(xb, wb, T, h, E, logits, st);
+    } else if (t.k == sgl::kSplit4) {
+      sgl::launch_router_ks<32, 32, 8>(xb, wb, T, h, E, logits, st);
+    } else {
+      sgl::launch_router_lds<32, 32, 8>(xb, wb, T, h, E, logits, st);
+    }
   } else if (T <= 256) {
     dim3 grid((unsigned)E / 16 + (E % 16 != 0), (unsigned)sgl::ceil_div(T, 16));
     sgl::router_logits_kernel<1, 1, 16, 8><<<grid, 1024, 0, st>>>(xb, wb, T, (int)H, E, logits);

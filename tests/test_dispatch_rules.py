@@ -27,6 +27,10 @@ int few(int64_t queries, int heads, int64_t K, int cus) { return attn_plan(queri
 int small_moe(int64_t T, int64_t H, int64_t I, int k, int shared, int fp4) {
   return small_moe_ok(T, H, I, k, shared, fp4, 256);
 }
+int router(int64_t T, int64_t H, int64_t E) {
+  const RouterTile t = router_tile(T, H, E);
+  return t.tokens * 10000 + t.experts * 10 + t.k;
+}
 int tall(int fp4, int64_t rows, int64_t tiles, int64_t cus) { return moe_tall_tiles(fp4, rows, tiles, cus); }
 int k_groups(int64_t M, int64_t N, int64_t K, int splits) { return dense_k_groups(M, N, K, splits); }
 }
@@ -139,3 +143,18 @@ def test_smallest_moe_batches_where_they_win(rules, fp4, T, H, I, k, small):
 def test_smallest_fp4_batches_without_a_shared_expert(rules, T, H, I, k, small):
     i64 = ctypes.c_int64
     assert rules.small_moe(i64(T), i64(H), i64(I), k, 0, 1) == small
+
+
+@pytest.mark.parametrize("T,H,E,tile", [
+    (512, 4096, 256, (32, 32, 1)), (512, 4160, 256, (32, 32, 0)), (2048, 4096, 256, (32, 64, 2)),
+    (2048, 7168, 256, (32, 64, 1)), (3700, 4096, 256, (32, 64, 1)), (3000, 2048, 256, (32, 64, 2)),
+    (3000, 4160, 256, (32, 64, 0)), (2048, 4160, 256, (32, 64, 2)), (4096, 4096, 256, (32, 128, 2)),
+    (4096, 2048, 256, (32, 128, 0)), (4097, 4096, 256, (64, 128, 2)), (8192, 4096, 256, (64, 128, 0)),
+    (16384, 4096, 256, (64, 128, 0)), (16384, 7168, 256, (64, 128, 2)), (16384, 7168, 128, (64, 128, 0)),
+    (2752, 4096, 384, (32, 128, 0)), (2880, 4096, 384, (64, 128, 2)),
+])
+def test_router_tiles_where_they_win(rules, T, H, E, tile):
+    """Tile and K split (0 one chain, 1 over four wavefronts, 2 groups) by both measured sides."""
+    i64 = ctypes.c_int64
+    got = rules.router(i64(T), i64(H), i64(E))
+    assert (got // 10000, got % 10000 // 10, got % 10) == tile
