@@ -747,8 +747,21 @@ __global__ __launch_bounds__(kPermThreads) void permute_place_kernel(
   all[tid] = sum;
   before[tid] = pre;
   __syncthreads();
+  // the parts of an expert: halved while there are many (few experts: with 1024
+  // parts read one after the other 16384 slots of one expert took 20.8 us, the
+  // four launches before 14.6), then one after the other
+  int n = parts;
+  while (n > 8) {
+    const int half = (n + 1) / 2;
+    if (tid < (n - half) * E) {
+      all[tid] = sum += all[tid + half * E];
+      before[tid] = pre += before[tid + half * E];
+    }
+    n = half;
+    __syncthreads();
+  }
   if (tid < E)
-    for (int q = 1; q < parts; ++q) {
+    for (int q = 1; q < n; ++q) {
       sum += all[q * E + tid];
       pre += before[q * E + tid];
     }
@@ -1028,13 +1041,8 @@ int check_moe_shapes(const char* what, int64_t T, int64_t H, int64_t I, int E, i
 // Also zeroes zero[0, nzero) (nzero <= 1024) on the way, for the caller's
 // tile counters.  Only the slots whose expert lies in [elo, ehi) are placed
 // (0 <= elo <= ehi <= E; the whole range for a layer on one rank).  table: P
-// ints of scratch that no output overlaps, or null.
-//
-// One workgroup or chunks (E = 256, k = 8, one workgroup / chunks with a table /
-// without): 2048 slots 6.5 / 7.1 / 8.7 us, 2400 8.0 / 7.3 / 8.7, 3072 8.5 / 7.4
-// / 8.7, 4096 10.4 / 7.5 / 9.0, 15200 31.7 / 8.5 / 9.9, 65536 126 / 8.9 / 10.4
-// (four launches over chunks of 4096 slots 20.3; 262144 37.1 / here 13.1).
-constexpr int kPermRounds = 2, kPermRoundsNoTable = 3;
+// ints of scratch that no output overlaps, or null.  One workgroup or chunks:
+// permute_rounds.
 int launch_permute(const int32_t* ids, int64_t T, int k, int E, int32_t* counts, int32_t* offsets,
                    int32_t* sorted_slot, int32_t* slot_pos, int32_t* zero, int nzero,
                    int32_t* table, hipStream_t st, int elo = 0, int ehi = -1) {
@@ -1049,7 +1057,7 @@ int launch_permute(const int32_t* ids, int64_t T, int k, int E, int32_t* counts,
               "moe_permute: null pointer");
   const int64_t P = T * k;
   const int64_t rounds = ceil_div(P, (int64_t)kPermThreads);
-  if (rounds <= (table ? kPermRounds : kPermRoundsNoTable)) {
+  if (rounds <= permute_rounds(E, table != nullptr)) {
     permute_kernel<<<1, kPermThreads, 0, st>>>(ids, P, E, counts, offsets, sorted_slot, slot_pos,
                                                zero, nzero, elo, ehi);
     return check_launch("moe_permute");

@@ -224,4 +224,16 @@ SGL_RULE RouterTile router_tile(int64_t T, int64_t H, int64_t E) {
   return {32, 32, even ? kSplit4 : kOneChain};
 }
 
+// ---- permute (counting sort of the slots by expert): rounds of 1024 slots that
+// one workgroup walks rather than chunks of them ranked and placed by many.  One
+// workgroup / chunks with a table / without, us:
+//   E = 256: 2048 slots 6.5 / 7.1 / 8.6, 2400 7.9 / 7.1 / 8.7, 3072 8.4 / 7.1 / 8.7,
+//     4096 10.3 / 7.4 / 8.9, 15200 31.7 / 8.5 / 9.9, 65536 126 / 8.9 / 10.4
+//   E = 32: 3072 7.1 / 6.7 / 8.4, 4096 8.5 / 6.8 / 8.4; E = 16: 2100 6.3 / 6.7 / 8.4, 3072
+//     6.9 / 6.8 / 8.4, 3600 8.0 / 6.7 / 8.3, 4096 8.4 / 6.8 / 8.4; E = 1024: 2400 9.9 /
+//     11.0 / 12.2
+SGL_RULE int permute_rounds(int E, bool table) {
+  return (table && E <= 512 ? 2 : 3) + (E <= (table ? 16 : 32) ? 1 : 0);
+}
+
 }  // namespace sgl

@@ -31,6 +31,7 @@ int router(int64_t T, int64_t H, int64_t E) {
   const RouterTile t = router_tile(T, H, E);
   return t.tokens * 10000 + t.experts * 10 + t.k;
 }
+int perm_rounds(int E, int table) { return permute_rounds(E, table); }
 int tall(int fp4, int64_t rows, int64_t tiles, int64_t cus) { return moe_tall_tiles(fp4, rows, tiles, cus); }
 int k_groups(int64_t M, int64_t N, int64_t K, int splits) { return dense_k_groups(M, N, K, splits); }
 }
@@ -158,3 +159,9 @@ def test_router_tiles_where_they_win(rules, T, H, E, tile):
     i64 = ctypes.c_int64
     got = rules.router(i64(T), i64(H), i64(E))
     assert (got // 10000, got % 10000 // 10, got % 10) == tile
+
+
+@pytest.mark.parametrize("E,table,rounds", [(256, 1, 2), (256, 0, 3), (32, 1, 2), (32, 0, 4), (8, 1, 3), (1, 0, 4),
+                                            (1024, 1, 3)])
+def test_permute_chunks_where_they_win(rules, E, table, rounds):
+    assert rules.perm_rounds(E, table) == rounds

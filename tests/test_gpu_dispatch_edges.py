@@ -256,6 +256,12 @@ def test_router_k_groups(gpu, T, H, E):
     (439, 7, 256),    # 3073: four chunks, one slot in the last
     (700, 6, 1024),   # chunks doubled so that their table fits in the slots, no idle expert thread
     (5000, 1, 1),     # one expert: every thread sums a part of the table
+    (4096, 1, 1),     # ... and the four rounds of one workgroup before
+    (70001, 1, 1),    # ... 69 chunks: more parts than chunks have
+    (140000, 1, 3),   # 341 parts, halved with an odd one left over
+    (40000, 2, 100),  # ten parts: one halving
+    (2048, 2, 8),     # eight experts: four rounds of one workgroup
+    (2049, 2, 8),     # ... and chunks
     (2001, 3, 1000),  # experts that do not divide the workgroup's threads
     (16385, 8, 200),  # chunks of two rounds
 ])
