@@ -194,15 +194,22 @@ def call(name: str, *args) -> None:
         check(status, name)
 
 
+# workspace sizes that are functions of their arguments alone (the sparse
+# attention's also depends on the current device's CU count)
+_PURE_SIZES = frozenset({"sgl_fp8_gemm_workspace_size", "sgl_moe_workspace_size"})
+
+
 @functools.lru_cache(maxsize=1024)
 def _size(lib, name: str, args: tuple) -> int:
     return int(getattr(lib, name)(*args))
 
 
 def size_of(name: str, *args: int) -> int:
-    """A ``sgl_*_workspace_size`` function: pure functions of the sizes, asked
-    on every call of their operation, so the last answers are kept."""
-    return _size(load(), name, args)
+    """A ``sgl_*_workspace_size`` function.  It is asked on every call of its
+    operation, so the last answers of those that are functions of the sizes
+    alone are kept."""
+    lib = load()
+    return _size(lib, name, args) if name in _PURE_SIZES else int(getattr(lib, name)(*args))
 
 
 def ptr(t) -> Optional[int]:

@@ -253,3 +253,27 @@ def test_fp8_gemm_split_decision_is_a_function_of_the_shape():
         rc = lib.sgl_fp8_gemm(fake, fake, 0, fake, fake, 0, fake, 0, 40, 4096, 7168, buf, n, None)
         assert rc == L.SGL_ERR_WORKSPACE, rc
         assert str(need) in L.last_error()
+
+
+def test_device_dependent_workspace_sizes_are_asked_each_time(monkeypatch):
+    """The sparse attention's workspace depends on the current device's CUs, so
+    its size is never a kept answer; sizes of shapes alone may be."""
+    from sglang_lite_amd import _lib
+
+    class Fake:
+        asked = 0
+
+        def sgl_sparse_attn_workspace_size(self, *args):
+            self.asked += 1
+            return 1000 * self.asked
+
+        def sgl_moe_workspace_size(self, *args):
+            self.asked += 1
+            return sum(args)
+
+    fake = Fake()
+    monkeypatch.setattr(_lib, "load", lambda: fake)
+    assert [_lib.size_of("sgl_sparse_attn_workspace_size", 1, 1, 8, 64) for _ in range(2)] == [1000, 2000]
+    fake.asked = 0
+    assert [_lib.size_of("sgl_moe_workspace_size", 1, 2, 3, 4, 5, 1) for _ in range(2)] == [16, 16]
+    assert fake.asked == 1
