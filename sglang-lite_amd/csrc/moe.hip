@@ -1275,8 +1275,6 @@ int sgl_moe_gate(const void* x, const void* w, int64_t T, int64_t H, int E, int 
     } else if (t.experts == 64) {
       if (t.k == sgl::kGroups)
         sgl::launch_router_lds<32, 64, 3, 4>(xb, wb, T, h, E, logits, st);
-      else if (t.k == sgl::kSplit4)
-        sgl::launch_router_ks<32, 64, 6>(xb, wb, T, h, E, logits, st);
       else
         sgl::launch_router_lds<32, 64, 6>(xb, wb, T, h, E, logits, st);
     } else if (t.k == sgl::kSplit4) {

@@ -188,21 +188,25 @@ SGL_RULE bool small_moe_ok(int64_t T, int64_t H, int64_t I, int k, int has_share
 // tile, and how its wavefronts share K.  The tiles are the largest that still
 // give about a workgroup per CU, 64 x 128 as soon as 32 x 128 are more than one
 // round of the 256 CUs (T = 6000, H = 4096, E = 256: 53 us in two rounds, 41 in
-// one; three columns of tiles share x so well that the few tiles past a round
-// fit beside it, one chain a workgroup, two workgroups a CU: T = 2752, E = 384,
-// 258 tiles 35 / 39).  K over the four wavefronts (kSplit4, H % 128 == 0) for the
-// 32-token tiles of 32 or 64 experts (T = 512 13.0 -> 9.4 us); over two or four
-// groups of four wavefronts with a 64-deep K block each (kGroups), whose chain
-// of stages is shorter, where it is the faster, E = 256, gate with them /
-// without:
-//   32 x 64 tiles: H = 2048, T = 2048 15.0 / 16.0 us, 3000 22.0 / 24.0; H = 4096, T =
-//     2048 18.5 / 19.9, 3700 39.0 / 38.1; H = 7168, T = 2048 33.1 / 31.7, 3000 57.0 /
-//     54.6; H = 4160, T = 2048 19.0 / 23.7, 3000 37.8 / 35.5
-//   32 x 128: H = 2048 22.0 / 22.3, 3072 28.5 / 28.3, 4096 32.7 / 33.2, 7168 47.8 / 48.8
-//   64 x 128: H = 2048, T = 4200 25.1 / 26.1, 12288 51.8 / 50.2; H = 4096, T = 4200
-//     39.2 / 39.5, 8192 44.7 / 44.6, 16384 90.0 / 87.0; H = 7168, T = 8192 64.4 /
-//     64.9, 16384 121.6 / 121.5; E = 160, T = 4640 32.6 / 35.4; E = 128, H = 4096, T =
-//     16384 53.8 / 51.4
+// one; but H = 1024, T = 4200 19.1 / 20.1, and three columns of tiles share x so
+// well that the few tiles past a round fit beside it, one chain a workgroup, two
+// workgroups a CU: T = 2752, E = 384, 258 tiles 35 / 39).  K over the four
+// wavefronts (kSplit4, H % 128 == 0) for the 32 x 32 tiles (T = 512 13.0 -> 9.4
+// us); for the larger ones over two or four groups of four wavefronts with a
+// 64-deep K block each (kGroups), whose chain of stages is shorter.  What they
+// save shows with x in the last-level cache, where the norm before the router
+// has left it; with x out of memory (here: inputs past 256 MB in turn) the tiles
+// wait for x, and some sizes lose a little.  E = 256, groups / without, x cached
+// and x out of memory, us:
+//   32 x 64 tiles: H = 2048, T = 3000 21.2 / 23.5 and 22.0 / 24.0; H = 4096, T = 2048
+//     18.5 / 19.8 both, 3700 30.1 / 32.5 and 39.0 / 38.1; H = 7168, T = 3000 42.0 / 44.3
+//     and 57.0 / 54.6; H = 4160, out of memory, T = 2048 19.0 / 23.7, 3000 37.8 / 35.5
+//   32 x 128: H = 1024 18.3 / 18.0, 4096 28.5 / 29.7 and 32.7 / 33.2, 7168 39.9 / 43.0
+//     and 47.8 / 48.8
+//   64 x 128: H = 1024, T = 16384 out of memory 44.2 / 42.1; H = 2048, T = 12288 44.6 /
+//     46.5 and 51.8 / 50.2; H = 4096, T = 6000 34.7 / 38.1 and 41.2 / 41.4, 8192 38.6 /
+//     41.5 and 44.7 / 44.6, 16384 70.6 / 76.7 and 90.0 / 87.0; H = 7168, T = 8192 53.3 /
+//     58.1 and 64.4 / 64.9; E = 128, H = 4096, T = 16384 39.6 / 40.8 and 53.8 / 51.4
 // (A tile's K in one chain errs by 4.0e-7 of the logits, in two by 2.7e-7, in
 // four by 1.9e-7, so no size goes to fewer chains than it had.)
 enum RouterK { kOneChain, kSplit4, kGroups };
@@ -214,13 +218,10 @@ SGL_RULE RouterTile router_tile(int64_t T, int64_t H, int64_t E) {
   const bool even = H % 128 == 0;
   const int64_t cols = (E + 127) / 128, rows = (T + 31) / 32;
   const int64_t t64 = rows * ((E + 63) / 64), t128 = rows * cols, tall = (T + 63) / 64 * cols;
-  if (t128 > (cols >= 3 ? 264 : 256))
-    return {64, 128, cols >= 2 && H >= 2048 && (H > 4160 || tall < 240) ? kGroups : kOneChain};
-  if (t128 >= 240) return {32, 128, even && cols >= 2 && H >= 4096 && t128 <= 256 ? kGroups : kOneChain};
-  if (t64 >= 240) {
-    if (even ? H <= 3072 || (H <= 4096 && t64 <= 256) : t64 <= 256) return {32, 64, kGroups};
-    return {32, 64, even ? kSplit4 : kOneChain};
-  }
+  if (t128 > (cols >= 3 ? 264 : 256) && (H >= 2048 || tall >= 240))
+    return {64, 128, H >= 2048 ? kGroups : kOneChain};
+  if (t128 >= 240) return {32, 128, H >= 2048 && t128 <= 256 ? kGroups : kOneChain};
+  if (t64 >= 240) return {32, 64, even || t64 <= 256 ? kGroups : kOneChain};
   return {32, 32, even ? kSplit4 : kOneChain};
 }
 

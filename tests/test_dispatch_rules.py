@@ -148,11 +148,10 @@ def test_smallest_fp4_batches_without_a_shared_expert(rules, T, H, I, k, small):
 
 @pytest.mark.parametrize("T,H,E,tile", [
     (512, 4096, 256, (32, 32, 1)), (512, 4160, 256, (32, 32, 0)), (2048, 4096, 256, (32, 64, 2)),
-    (2048, 7168, 256, (32, 64, 1)), (3700, 4096, 256, (32, 64, 1)), (3000, 2048, 256, (32, 64, 2)),
-    (3000, 4160, 256, (32, 64, 0)), (2048, 4160, 256, (32, 64, 2)), (4096, 4096, 256, (32, 128, 2)),
-    (4096, 2048, 256, (32, 128, 0)), (4097, 4096, 256, (64, 128, 2)), (8192, 4096, 256, (64, 128, 0)),
-    (16384, 4096, 256, (64, 128, 0)), (16384, 7168, 256, (64, 128, 2)), (16384, 7168, 128, (64, 128, 0)),
-    (2752, 4096, 384, (32, 128, 0)), (2880, 4096, 384, (64, 128, 2)),
+    (2048, 7168, 256, (32, 64, 2)), (3700, 4096, 256, (32, 64, 2)), (3000, 4160, 256, (32, 64, 0)),
+    (2048, 4160, 256, (32, 64, 2)), (4096, 4096, 256, (32, 128, 2)), (4096, 1024, 256, (32, 128, 0)),
+    (4097, 4096, 256, (64, 128, 2)), (4200, 1024, 256, (32, 128, 0)), (8192, 4096, 256, (64, 128, 2)),
+    (8192, 1024, 256, (64, 128, 0)), (2752, 4096, 384, (32, 128, 0)), (2880, 4096, 384, (64, 128, 2)),
 ])
 def test_router_tiles_where_they_win(rules, T, H, E, tile):
     """Tile and K split (0 one chain, 1 over four wavefronts, 2 groups) by both measured sides."""

@@ -224,12 +224,11 @@ def test_sparse_attn_moving_reference(gpu, order):
     (1921, 320, 256),   # 32 x 64 tiles, 5 K blocks for four groups
     (2049, 64, 248),    # 32 x 64 tiles, one K block: three groups have none
     (1920, 384, 256),   # 32 x 64 tiles from here (240), 6 K blocks
-    (1921, 3200, 256),  # ... past H = 3072 in one round
-    (2049, 3200, 256),  # ... and in two: the four-way split's 32 x 64 tiles
     (2049, 192, 256),   # an odd number of K blocks in two rounds: one chain
-    (4096, 4096, 256),  # 32 x 128 tiles, two groups
-    (7680, 256, 256),   # 64 x 128 tiles from 240 of them: one chain
-    (7679, 4224, 250),  # ... below, two groups
+    (4096, 2048, 256),  # 32 x 128 tiles, two groups
+    (4097, 2112, 250),  # 64 x 128 tiles, two groups, 33 K blocks
+    (7680, 256, 256),   # 64 x 128 tiles of short rows: one chain
+    (7679, 256, 250),   # ... 32 x 128 below 240 of them
     (2752, 256, 320),   # three columns of 32 x 128 tiles a little past one round
     (1919, 384, 192),   # the four-way split's 32 x 32 tiles
 ])
