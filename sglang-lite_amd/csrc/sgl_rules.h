@@ -55,14 +55,16 @@ SGL_RULE AttnMerge attn_merge_at(uint32_t wg, uint32_t wave, uint32_t queries, u
 // per 64 heads) that a merge reads back; attn_few.hip (at most 64 heads) starts
 // sooner than attn.hip but is slower a block.  The cheapest by these costs, in
 // 1/100 us, fitted to 1 ... 256 queries x 64 ... 2048 indices x 1 ... 128 heads,
-// bf16 rows and packed pages, both kernels, every number of splits:
+// all valid, bf16 rows and packed pages, both kernels, every number of splits
+// (the choice is within 0.4 % of the best for each shape and format on average;
+// one choice for both formats costs bf16 rows up to about 13 %):
 //   a block of 64 indices: 250 (attn.hip, whose own blocks are 32 rows: at most
 //     32 indices 125);
-//   attn_few.hip against attn.hip: 75 a block more, and to start 285 - 3.6 heads
-//     less (at most 32 heads) or 150 - 2.4 (heads - 32) less;
-//   a merge: 140 and 31 a split, up to 88 more with the heads, and for each
+//   attn_few.hip against attn.hip: 75 a block more, and to start 288 - 4 heads
+//     less (at most 32 heads) or 185 - 4.7 (heads - 32) less;
+//   a merge: 250 and 31 a split, up to 74 more with the heads, and for each
 //     partial of 64 heads 4.5 where the merge follows its splits (a multiple of
-//     eight queries), else 7.2, at most 990.
+//     eight queries), else 8, at most 900.
 // (Packed pages, us.  64 heads: 32 / 33 queries x 128 indices, one split / two
 // 15.2 / 17.4 and 15.1 / 20.7; 32 x 384, one / three 25.3 / 20.8; 32 x 640, one
 // / five 35.6 / 23.5; 33 x 2048, seven 36.7, eight, which are 264 workgroups,
@@ -82,15 +84,15 @@ SGL_RULE AttnPlan attn_plan(int64_t queries, int heads, int64_t K, int cus) {
   int64_t best_cost = K <= 32 ? 125 : blocks * 250;
   for (int kernel = 0; kernel < (heads <= 64 ? 2 : 1); ++kernel) {
     const bool few = kernel == 1;
-    const int64_t start = !few ? 0 : heads <= 32 ? 285 - 36 * heads / 10 : 150 - 24 * (heads - 32) / 10;
+    const int64_t start = !few ? 0 : heads <= 32 ? 288 - 4 * heads : 185 - 47 * (heads - 32) / 10;
     for (int64_t want = 1; want <= kAttnMaxSplits && (want == 1 || (want <= blocks && want * wgs <= cus)); ++want) {
       const int64_t bps = (blocks + want - 1) / want;
       const int64_t ns = bps > 0 ? (blocks + bps - 1) / bps : 1;  // no empty split
       int64_t cost = (!few && K <= 32 ? 125 : bps * (few ? 325 : 250)) - start;
       if (ns > 1) {
-        int64_t parts = queries * ns * heads * (queries % 8 == 0 ? 45 : 72) / 640;
-        if (queries % 8 != 0 && parts > 990) parts = 990;
-        cost += 140 + 31 * ns + 88 * h64 / 64 + parts;
+        int64_t parts = queries * ns * heads * (queries % 8 == 0 ? 45 : 80) / 640;
+        if (queries % 8 != 0 && parts > 900) parts = 900;
+        cost += 250 + 31 * ns + 74 * h64 / 64 + parts;
       }
       if (cost < best_cost) {
         best_cost = cost;
