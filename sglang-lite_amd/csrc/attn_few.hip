@@ -167,10 +167,14 @@ void sparse_attn_few_kernel(const AttnArgs a) {
 
   const int nblk_all = (int)((a.K + kBlk - 1) / kBlk);
   const int jb = split * a.bps;  // this split's first block
-  const int nblk = jb + a.bps < nblk_all ? jb + a.bps : nblk_all;
+  int nblk = jb + a.bps < nblk_all ? jb + a.bps : nblk_all;
   // indices run two blocks ahead of the MFMAs, the rows one block ahead;
   // past the last block the loads repeat it (their results are unused)
-  int32_t ids = jb < nblk ? check_id(jb, load_ids(jb)) : -1;
+  int32_t ids = jb < nblk ? load_ids(jb) : -1;
+  // blocks at the end with every entry masked are left out (not those between
+  // others: a branch in the loop would split its loads)
+  while (nblk > jb + 1 && __ballot(check_id(nblk - 1, load_ids(nblk - 1)) >= 0) == 0) --nblk;
+  ids = check_id(jb, ids);
   int32_t ids_next = jb < nblk ? load_ids(jb + 1 < nblk ? jb + 1 : jb) : -1;  // raw (none when K == 0)
   load_rows(ids);
   // Q^T B operand: lane (head c32, half g2) of step ks holds

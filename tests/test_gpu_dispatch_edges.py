@@ -164,8 +164,10 @@ def test_sparse_attn_row_counts_at_block_edges(gpu, H, fmt):
 @pytest.mark.parametrize("fmt,K", [("bf16", 2752), ("bf16", 2753), ("rows", 1792), ("pages", 1793)])
 @pytest.mark.parametrize("queries", [1, 300])
 def test_sparse_attn_row_list_edges(gpu, fmt, K, queries):
-    """Selections that fill the row list of a workgroup exactly and by one more
-    (300 queries: unsplit; one: split, shorter lists)."""
+    """As many indices as the row list of a workgroup holds rows, and one more,
+    every seventh masked (300 queries: unsplit; one: split, a list each; lists
+    filled exactly and past their end by valid rows:
+    test_sparse_attn_row_lists_by_valid_rows)."""
     rng = np.random.default_rng(K)
     print(f"attn list K={K} queries={queries} {fmt}", flush=True)
     q, kv = bf16_values(rng, (1, queries, 2, 512)), bf16_values(rng, (1, 40, 512))
@@ -181,8 +183,9 @@ def test_sparse_attn_row_list_edges(gpu, fmt, K, queries):
 @pytest.mark.parametrize("queries", [8, 9, 24])
 @pytest.mark.parametrize("H", [6, 64, 70])
 def test_sparse_attn_merge_order(gpu, queries, H):
-    """Split rows merged on both orders of workgroups (a multiple of eight
-    queries or not), head counts that do not fill a workgroup's four."""
+    """The values of split rows merged in both orders of workgroups (a multiple
+    of eight queries or not), head counts that do not fill a workgroup's four
+    (where each merge runs: test_dispatch_rules.py)."""
     rng = np.random.default_rng(queries + H)
     K = 1024
     print(f"attn merge H={H} queries={queries}", flush=True)
@@ -355,3 +358,23 @@ def test_sparse_attn_short_chains(gpu, H, K, fmt):
         got, rows = _attn(gpu, q, kv, sink, idx, 512 ** -0.5, fmt)
         assert_gemm_close(got, OA.sparse_attn_blocked(q, rows, sink, idx, 512 ** -0.5), f"H={H} K={K} {fmt} {B}x{S}")
         assert np.all(got[0, 0] == 0)
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "pages"])
+@pytest.mark.parametrize("H,K", [(8, 64), (8, 130), (16, 192), (8, 640), (40, 64)])
+def test_sparse_attn_few_heads_masked_blocks(gpu, H, K, fmt):
+    """The kernel of few heads where whole blocks of 64 indices are masked: at
+    the end (left out), at the head, between others, everywhere."""
+    rng = np.random.default_rng(H + K)
+    print(f"attn masked blocks H={H} K={K} {fmt}", flush=True)
+    n, S = 90, 9
+    q, kv = bf16_values(rng, (1, S, H, 512)), bf16_values(rng, (1, n, 512))
+    sink = rng.standard_normal(H).astype(np.float32)
+    idx = rng.integers(0, n, (1, S, K)).astype(np.int32)
+    for s, keep in enumerate((0, 1, 63, 64, 65, K - 1, K)):  # a prefix of valid entries
+        idx[0, s, keep:] = -1
+    idx[0, 7, :K - 1] = -1
+    idx[0, 8, 1:K - 1] = -1
+    got, rows = _attn(gpu, q, kv, sink, idx, 512 ** -0.5, fmt)
+    assert_gemm_close(got, OA.sparse_attn_blocked(q, rows, sink, idx, 512 ** -0.5), f"H={H} K={K} {fmt}")
+    assert np.all(got[0, 0] == 0)
