@@ -16,12 +16,16 @@
 // exact in bf16; v_cvt_scalef32_pk_bf16_fp8 rounds it exactly), so the packed
 // cache feeds the attention with no bf16 copy of it in HBM.
 //
-// One workgroup per (query token, group of 64 heads, split of the rows); a
-// small batch (decode) splits its rows over several workgroups so every CU
-// has one, and a second kernel merges the splits' partial maxima, sums and
-// outputs.  The split's valid indices are packed into a list in LDS first, so
-// masked entries (-1 pads of a short context, a prefill's early queries) cost
-// nothing.  Eight wavefronts in two roles, one of each per SIMD, so one
+// One workgroup per (query token, group of 64 heads, split of the indices); a
+// small batch (decode) splits its indices over several workgroups, at most one
+// a CU, and a second kernel merges the splits' partial maxima, sums and
+// outputs (the rules, and the few heads and short chains that attn_few.hip
+// takes: attn_plan in sgl_rules.h).  The split's valid indices are packed into
+// a list in LDS first, so the masked entries of a call of one split (a
+// prefill's early queries) cost only their index.  A split is a range of
+// index positions: where they are all masked (the -1 pads at the end of a short
+// context) its workgroup has no rows but still writes its partial.
+// Eight wavefronts in two roles, one of each per SIMD, so one
 // role's MFMAs fill the other's waits; the roles run blocks of 32 rows in
 // phases with one barrier each, S^T of block j + 1 beside O^T of block j:
 //   gather:  wavefronts 4-7, 8 rows each, into a ring of four 32 KB row-major
@@ -45,10 +49,10 @@
 // V^T reads and 16 KB of P reads; each SIMD 1024 cycles of MFMA (0.7 of the
 // 1.1 us a block takes), and a workgroup fills a CU, so its first loads and
 // its output rows (about 7 us a query) stand alone.  256 queries x 640 /
-// 2048 rows of a bf16 cache 45.9 / 113 -> 34.2 / 81 us against the version
+// 2048 rows of a bf16 cache 45.1 / 104 -> 34.0 / 73.6 us against the version
 // before (one role, S^T over split dims with partial sums through LDS, 64-row
-// blocks), packed pages 53 / 133 -> 41.5 / 105; a 2048-token prefill chunk
-// (640 indices, -1 where a token has fewer rows) 320 -> 182 us.  The roles
+// blocks), packed pages 49.8 / 131 -> 37.7 / 92.2; a 2048-token prefill chunk
+// (640 indices, -1 where a token has fewer rows) 321 -> 183 us.  The roles
 // without the MFMAs between reads and gathers (each fragment read waited for
 // by itself): 1.3 us a block.
 #include "sgl_attn.h"
@@ -262,7 +266,8 @@ __device__ __forceinline__ void attn_role(const AttnArgs& a, Smem<FMT>& sm) {
     // their scale byte, and one load for the 16-byte rope pieces of all eight
     // rows (lane: row lane / 8, piece lane % 8).  (One row a load, 56 lanes x
     // 8 bytes, with the scales passed between lanes, took three times the
-    // instructions: 2048 rows x 256 queries 118 us, this form 105)
+    // instructions: 2048 rows x 256 queries 118 us against 105, both before
+    // the loads were global ones)
     int ln = lane;  // made opaque where the gathers run, so that their per-row offsets are formed there
                     // and not kept in registers across the phases
     auto dma_row = [&](int j, int rr, uint64_t row) {  // (a block past the last: nothing)

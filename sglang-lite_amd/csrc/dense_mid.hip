@@ -3,8 +3,8 @@
 //
 // C[M, N] = sum_kb (A[:, kb] . B[:, kb]^T) sa[m, kb] sb[n/128, kb], as
 // gemm_fp8_kernel computes it.  What bounds those tiles at M = 65 ... 512 is
-// neither memory (84 % of their reads hit L2) nor the matrix cores (10 % busy)
-// but the serial chain of a 128-deep stage (wait, barrier, fragment reads,
+// neither memory (M = 200, N = 4096, K = 7168: 84 % of their reads hit L2) nor
+// the matrix cores (busy 9 % of the time) but the serial chain of a 128-deep stage (wait, barrier, fragment reads,
 // MFMAs, promotion, the next loads' issue: about 1070 cycles at one workgroup
 // of four wavefronts a CU), 56 times over at K = 7168.  So here a stage holds
 // G K blocks, each computed by four wavefronts of its own over the whole tile,
@@ -16,8 +16,8 @@
 // N = 4096, K = 7168, e8m0 scales, graph-replayed over cold weights, the tiles
 // before (32 x 64 ... 64 x 128, one K block a stage) / these: M = 128 19.1 / 12.2
 // us (the weight alone reads in 7), 200 26.5 / 18.8, 512 40.0 / 26.1; N = 512:
-// M = 512 39.1 / 12.0, 4096 (256 x 256 tiles) 84 / 27; K = 2048, N = 4096: M = 128
-// 8.2 / 6.3, 512 15.4 / 10.6; fp32 scales, M = 128 / 512 21.4 / 13.1 and 35.2 / 30.0.
+// M = 512 39.1 / 12.0; K = 2048, N = 4096: M = 128 8.2 / 6.3, 512 15.4 / 10.6; fp32
+// scales, M = 128 / 200 / 512 21.4 / 13.1, 28.3 / 23.2 (by the trace) and 35.2 / 30.0.
 #include "sgl_gemm.h"
 #include "sgl_dense_mid.h"
 #include "sgl_numeric.h"
@@ -231,7 +231,10 @@ int launch_dense_mid(GemmArgs& a, hipStream_t st) {
   if (kb <= 64 && tiles(32, 64) <= cus) return launch_mid<MidCfg<32, 64, 4, 3, 64>>(a, st);
   if (kb <= 64 && tiles(32, 128) <= cus) return launch_mid<MidCfg<32, 128, 2, 3, 64>>(a, st);
   // up to three tiles a CU where the 256 x 256 tiles that would take the
-  // product (M > 2048) leave half the CUs or more without one
+  // product (M > 2048) leave half the CUs or more without one: M = 4096, K =
+  // 7168, those tiles / these, e8m0 and fp32 scales: N = 512 (one round) 84.1 /
+  // 28.6 and 96.8 / 33.7 us, 1024 (two) 85.5 / 54.0 and 101 / 63.8, 1536 (three)
+  // 89.9 / 81.0 and 106 / 92.8; K = 2048, N = 1536 35.0 / 30.7 and 38.6 / 34.7
   const bool few = a.M > 2048 && tiles(256, 256) <= cus / 2;
   if (kb <= 56 && tiles(64, 128) <= (few ? 3 * cus : cus)) return launch_mid<MidCfg<64, 128, 2, 3, 56>>(a, st);
   return kNoMid;

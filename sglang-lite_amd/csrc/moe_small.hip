@@ -25,8 +25,11 @@
 // h, 1x128 e4m3 h, bf16 expert outputs, fp32 sum in ascending expert id);
 // each product's K is summed per line, then over lines in order.
 //
-// H = 4096, I = 2048, top-8 + shared, E = 256, one token: FP4 73.0 -> 38.8 us,
-// FP8 68.0 -> 58.0 us.
+// H = 4096, I = 2048, top-8 + shared, E = 256, one token, the layer with its
+// activation quant, graph-replayed over cold weights: FP4 74.3 -> 41.3 us (gate/up
+// 22.2, down 16.8 by the trace), FP8 65.5 -> 57.8 (32.1 and 22.4, where the two
+// grouped launches took 33.0 and 20.3: only the permute and the combine are
+// saved, so the rule small_moe_ok in sgl_rules.h ends early for FP8).
 #include <algorithm>
 
 #include "sgl_gemm.h"
